@@ -143,12 +143,13 @@ PF_DEVICE float dpp_sum16(float v) {
   v += dpp_mov<0x140>(v);
   return v;
 }
-// Sum over aligned groups of W lanes, W in {16, 32}: DPP inside rows, one swizzle across.
+// Sum over aligned groups of W lanes, W in {16, 32, 64}: DPP inside rows, swizzles across.
 template <int W>
 PF_DEVICE float row_group_sum(float v) {
-  static_assert(W == 16 || W == 32, "row groups of 16 or 32 lanes");
+  static_assert(W == 16 || W == 32 || W == 64, "row groups of 16, 32 or 64 lanes");
   v = dpp_sum16(v);
-  if (W == 32) v += __shfl_xor(v, 16, 64);
+  if (W >= 32) v += __shfl_xor(v, 16, 64);
+  if (W == 64) v += __shfl_xor(v, 32, 64);
   return v;
 }
 

@@ -762,7 +762,9 @@ __global__ __launch_bounds__(256) void trimul_project32_kernel(const TZ* __restr
 // and gate rows of one channel land in one lane (accumulator rows r and r + 16), so the
 // gating is in registers; the gated values go through a double-buffered LDS stage
 // [a | b][16 channels][128 positions] and leave as 256-byte plane-row pieces one chunk later.
-// One barrier per chunk. (Three stages, weights two chunks ahead with each wait counting the
+// One barrier per chunk. An fp32 stream takes the same kernel without the prefetch (its half
+// row alone is 128 registers; rows past N are clamped, not skipped, because conditional loads
+// into that many registers spill): 481 -> 263 us against the tile kernel at N=500. (Three stages, weights two chunks ahead with each wait counting the
 // vector-memory operations issued after them, measured slower: 533 -> 600-609 us at N=768;
 // so did 64 positions per wave, whose operands spill.)
 struct Project256 {
@@ -840,16 +842,22 @@ __global__ __launch_bounds__(Project256::NT, 1) void trimul_project256_kernel(
     int b, line, t0;
     tile_pos(tl, b, line, t0);
     const int t = t0 + 32 * pb + lq;
-    const TZ* src = nullptr;
-    if (line < N && t < N)
-      src = z + ((size_t)b * N * N + (outgoing ? (long)line * N + t : (long)t * N + line)) * C + 8 * hf;
+    if constexpr (sizeof(TZ) == 2) {
+      const TZ* src = nullptr;
+      if (line < N && t < N)
+        src = z + ((size_t)b * N * N + (outgoing ? (long)line * N + t : (long)t * N + line)) * C + 8 * hf;
 #pragma unroll
-    for (int ks = 0; ks < C / 16; ++ks) {
-      if constexpr (sizeof(TZ) == 2) {
+      for (int ks = 0; ks < C / 16; ++ks)
         zr[ks] = src ? *reinterpret_cast<const u32x4*>(src + 16 * ks) : u32x4{0u, 0u, 0u, 0u};
-      } else {
-        zr[2 * ks] = src ? *reinterpret_cast<const u32x4*>(src + 16 * ks) : u32x4{0u, 0u, 0u, 0u};
-        zr[2 * ks + 1] = src ? *reinterpret_cast<const u32x4*>(src + 16 * ks + 4) : u32x4{0u, 0u, 0u, 0u};
+    } else {
+      // a row past N reads the last one and is zeroed where it is used: conditional loads
+      // of 128 registers spill
+      const int lc = min(line, N - 1), tc = min(t, N - 1);
+      const TZ* src = z + ((size_t)b * N * N + (outgoing ? (long)lc * N + tc : (long)tc * N + lc)) * C + 8 * hf;
+#pragma unroll
+      for (int ks = 0; ks < C / 16; ++ks) {
+        zr[2 * ks] = *reinterpret_cast<const u32x4*>(src + 16 * ks);
+        zr[2 * ks + 1] = *reinterpret_cast<const u32x4*>(src + 16 * ks + 4);
       }
     }
   };
@@ -880,7 +888,7 @@ __global__ __launch_bounds__(Project256::NT, 1) void trimul_project256_kernel(
   long tile = blockIdx.x;
   int sb = 0, sline = 0, st0 = 0;  // tile of the chunk waiting in the stage
   if (total > 0) {
-    load_half(tile);
+    if (PREFETCH) load_half(tile);
     for (int i = 0; i < NS - 1 && i < total; ++i) issue_chunk(i);
   }
   __syncthreads();  // LN parameters
@@ -892,7 +900,7 @@ __global__ __launch_bounds__(Project256::NT, 1) void trimul_project256_kernel(
     const bool live = line < N && tpos < N;
     const float mk =
         live ? mask[(size_t)b * N * N + (outgoing ? (long)line * N + tpos : (long)tpos * N + line)] : 0.f;
-    if (!PREFETCH && tile != (long)blockIdx.x) load_half(tile);
+    if (!PREFETCH) load_half(tile);
 
     // ---- LN (or the given x) -> B operands xf[ks]: channels 16 ks + 8 hf .. +7
     bf16x8 xf[C / 16];
@@ -926,7 +934,12 @@ __global__ __launch_bounds__(Project256::NT, 1) void trimul_project256_kernel(
         get(ks, v);
         const float* pw = lnp + 16 * ks + 8 * hf;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) xf[ks][e] = (bf16)((v[e] - mean) * rstd * pw[e] + pw[C + e]);
+        for (int e = 0; e < 8; ++e) {
+          const float y = (v[e] - mean) * rstd * pw[e] + pw[C + e];
+          xf[ks][e] = (bf16)(sizeof(TZ) == 2 || live ? y : 0.f);
+        }
+        // fp32 rows fill half the registers: the parameter reads of later pieces stay below
+        if (sizeof(TZ) == 4) __builtin_amdgcn_sched_barrier(0);
       }
     } else {
 #pragma unroll
@@ -934,7 +947,7 @@ __global__ __launch_bounds__(Project256::NT, 1) void trimul_project256_kernel(
         float v[8];
         get(ks, v);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) xf[ks][e] = (bf16)v[e];
+        for (int e = 0; e < 8; ++e) xf[ks][e] = (bf16)(sizeof(TZ) == 2 || live ? v[e] : 0.f);
       }
     }
     const bool more = tile + gridDim.x < ntiles;
@@ -1365,7 +1378,7 @@ __global__ __launch_bounds__(OutputWs::NT) void trimul_output_ws_kernel(
   }
 }
 
-// K3 at 256 channels, persistent and weight-stationary (bf16 GEMMs, bf16 z). One 512-thread
+// K3 at 256 channels, persistent and weight-stationary (bf16 GEMMs). One 512-thread
 // block per CU walks tiles of 64 positions (i, j0 .. j0+63) of one row. Wave w owns output
 // channels 32 w .. +32 for both position halves: its rows of out_proj and out_gate stay in
 // registers for the whole launch as 32x32x16 MFMA A operands (128 VGPRs), so no weight
@@ -1373,7 +1386,8 @@ __global__ __launch_bounds__(OutputWs::NT) void trimul_output_ws_kernel(
 // one tile ahead) goes to LDS and is normalised (LN_out) by a pass whose reads run along
 // positions; the z rows (also one tile ahead) are normalised (LN_in) from registers that
 // keep them for the residual; each 32-position half then runs 32 MFMAs per wave, stages its
-// fp32 update block-wide and adds it to the z rows of that half.
+// fp32 update block-wide and adds it to the z rows of that half. With fp32 z the residual
+// rows are read again instead of kept: 394 -> 217 us against the tile kernel at N=500.
 struct Output256 {
   static constexpr int C = 256;
   static constexpr int BP = 64;
@@ -1384,18 +1398,21 @@ struct Output256 {
   static constexpr int SLD = C + 4;   // fp32 update stage rows [pos][ch], one half tile
 };
 
+template <class TZ>
 __global__ __launch_bounds__(Output256::NT, 1) void trimul_output256_kernel(
-    const bf16* __restrict__ X, const bf16* __restrict__ z, bf16* __restrict__ out, const float* __restrict__ lniw,
+    const bf16* __restrict__ X, const TZ* __restrict__ z, TZ* __restrict__ out, const float* __restrict__ lniw,
     const float* __restrict__ lnib, float eps_in, const float* __restrict__ lnow, const float* __restrict__ lnob,
     float eps_out, const bf16* __restrict__ Wo, const bf16* __restrict__ Wog, int B, int N, int Np, int accumulate) {
   using Cfg = Output256;
   constexpr int C = Cfg::C, BP = Cfg::BP, NW = Cfg::NW, NT = Cfg::NT, XLD = Cfg::XLD, TLD = Cfg::TLD,
                 SLD = Cfg::SLD;
-  constexpr int VEC = 8;                 // z elements per 16-byte load
-  constexpr int LPR = C / VEC;           // lanes per z row (32)
-  constexpr int RPI = 64 / LPR;          // z rows per wave-wide load (2)
+  constexpr bool PARK = sizeof(TZ) == 2;  // bf16 z rows wait for the residual in LDS
+  constexpr int ES = (int)sizeof(TZ);
+  constexpr int VEC = 16 / ES;           // z elements per 16-byte load
+  constexpr int LPR = C / VEC;           // lanes per z row (32; fp32 z: 64)
+  constexpr int RPI = 64 / LPR;          // z rows per wave-wide load (2; 1)
   constexpr int RPW = BP / NW;           // z rows per wave per tile (8)
-  constexpr int NLD = RPW / RPI;         // z loads per lane per tile (4)
+  constexpr int NLD = RPW / RPI;         // z loads per lane per tile (4; 8)
   constexpr int XLDS = C * BP / 8 / NT;  // 16-byte X loads per lane per tile (4)
   __shared__ __attribute__((aligned(16))) bf16 xt[C * TLD];   // X tile [ch][pos]
   __shared__ __attribute__((aligned(16))) bf16 xa[BP * XLD];  // LN_out(X) [pos][ch]
@@ -1446,14 +1463,20 @@ __global__ __launch_bounds__(Output256::NT, 1) void trimul_output256_kernel(
   // spill reload waited for the next tile's loads in flight. The z rows' buffer ends at
   // position N of the row, so rows past N load zeros and their stores are dropped.
   u32x4 zr[NLD], xr[XLDS];
-  auto issue = [&](int tile) {
+  auto z_row_rsrc = [&](int b, int i, int j0) {
+    return buf_rsrc(z + (((size_t)b * N + i) * N + j0) * C, (unsigned)((N - j0) * C * ES));
+  };
+  auto issue_z = [&](int tile) {
     int b, i, j0;
     tile_coords(tile, b, i, j0);
-    const __amdgpu_buffer_rsrc_t zrs =
-        buf_rsrc(z + (((size_t)b * N + i) * N + j0) * C, (unsigned)((N - j0) * C * 2));
+    const __amdgpu_buffer_rsrc_t zrs = z_row_rsrc(b, i, j0);
 #pragma unroll
     for (int q = 0; q < NLD; ++q)
-      zr[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(zrs, (zoff0 + q * RPI * C) * 2, 0, 0));
+      zr[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(zrs, (zoff0 + q * RPI * C) * ES, 0, 0));
+  };
+  auto issue_x = [&](int tile) {
+    int b, i, j0;
+    tile_coords(tile, b, i, j0);
     const __amdgpu_buffer_rsrc_t xrs = buf_rsrc(X + (size_t)b * C * pe, (unsigned)((size_t)C * pe * 2));
 #pragma unroll
     for (int q = 0; q < XLDS; ++q)
@@ -1462,10 +1485,15 @@ __global__ __launch_bounds__(Output256::NT, 1) void trimul_output256_kernel(
                      xrs, (int)((unsigned)(i * Np + j0 + q * (NT / 8) * pe + xoff) * 2u), 0, 0));
   };
 
-  // After the LN_out pass the X tile's LDS holds the raw z rows [pos][ch] for the residual.
+  // bf16 z: after the LN_out pass the X tile's LDS holds the raw z rows [pos][ch] for the
+  // residual. fp32 rows do not fit there (64 KB): the residual pass reads its rows again (the
+  // tile's own, a few microseconds old in L2) before it overwrites them.
   bf16* zs = xt;
   int tile = blockIdx.x;
-  if (tile < ntiles) issue(tile);
+  if (tile < ntiles) {
+    issue_z(tile);
+    issue_x(tile);
+  }
   __syncthreads();  // LN parameters
   for (; tile < ntiles; tile += gridDim.x) {
     int b, i, j0;
@@ -1480,7 +1508,7 @@ __global__ __launch_bounds__(Output256::NT, 1) void trimul_output256_kernel(
 #pragma unroll
     for (int q = 0; q < NLD; ++q) {
       float zv[VEC];
-      unpack16<bf16>(zr[q], zv);
+      unpack16<TZ>(zr[q], zv);
       float sum = 0.f;
 #pragma unroll
       for (int e = 0; e < VEC; ++e) sum += zv[e];
@@ -1521,14 +1549,19 @@ __global__ __launch_bounds__(Output256::NT, 1) void trimul_output256_kernel(
     }
     __syncthreads();  // xa, xb complete; every wave is done with the X tile
     // raw z rows -> zs (each lane reads back only what it wrote), then the next tile's loads
+    if constexpr (PARK) {
 #pragma unroll
-    for (int q = 0; q < NLD; ++q)
-      *reinterpret_cast<u32x4*>(zs + (w * RPW + q * RPI + l / LPR) * C + chunk * VEC) = zr[q];
+      for (int q = 0; q < NLD; ++q)
+        *reinterpret_cast<u32x4*>(zs + (w * RPW + q * RPI + l / LPR) * C + chunk * VEC) = zr[q];
+    }
     const int next = tile + gridDim.x;
-    if (next < ntiles) issue(next);
+    if (next < ntiles) {
+      issue_z(next);
+      issue_x(next);
+    }
 
     const __amdgpu_buffer_rsrc_t ors =
-        buf_rsrc(out + (((size_t)b * N + i) * N + j0) * C, (unsigned)((N - j0) * C * 2));
+        buf_rsrc(out + (((size_t)b * N + i) * N + j0) * C, (unsigned)((N - j0) * C * ES));
 #pragma unroll 1
     for (int pt = 0; pt < 2; ++pt) {
       f32x16 ao, ag;
@@ -1559,17 +1592,32 @@ __global__ __launch_bounds__(Output256::NT, 1) void trimul_output256_kernel(
         for (int q = 0; q < NLD; ++q) {
           const int p = w * RPW + q * RPI + l / LPR;
           float zv[VEC], y[VEC];
-          unpack16<bf16>(*reinterpret_cast<const u32x4*>(zs + p * C + chunk * VEC), zv);
+          if constexpr (PARK) {
+            unpack16<bf16>(*reinterpret_cast<const u32x4*>(zs + p * C + chunk * VEC), zv);
+          } else {
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) zv[e] = 0.f;
+            if (accumulate)
+              unpack16<TZ>(__builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                         z_row_rsrc(b, i, j0), (p * C + chunk * VEC) * ES, 0, 0)),
+                           zv);
+          }
 #pragma unroll
           for (int e = 0; e < VEC; e += 4) {
             const f32x4 u = *reinterpret_cast<const f32x4*>(upd + (p - 32 * pt) * SLD + chunk * VEC + e);
 #pragma unroll
             for (int k = 0; k < 4; ++k) y[e + k] = accumulate ? zv[e + k] + u[k] : u[k];
           }
-          bf16x8 o8;
+          u32x4 o;
+          if constexpr (PARK) {
+            bf16x8 o8;
 #pragma unroll
-          for (int e = 0; e < VEC; ++e) o8[e] = (bf16)y[e];
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o8), ors, (p * C + chunk * VEC) * 2, 0, 0);
+            for (int e = 0; e < VEC; ++e) o8[e] = (bf16)y[e];
+            o = __builtin_bit_cast(u32x4, o8);
+          } else {
+            o = __builtin_bit_cast(u32x4, f32x4{y[0], y[1], y[2], y[3]});
+          }
+          __builtin_amdgcn_raw_buffer_store_b128(o, ors, (p * C + chunk * VEC) * ES, 0, 0);
         }
       }
     }
@@ -1732,8 +1780,8 @@ __global__ void trimul_pack_kernel(const TS* __restrict__ wp, const TS* __restri
 }
 
 // C = 128 in bf16 runs the persistent weight-stationary K1/K3 and C = 256 with bf16 z the
-// persistent weight-streaming K1; fp32 and the other channel counts (the template stack's 64)
-// run the generic tile kernels, as does K3 at 256 channels.
+// persistent weight-streaming K1 and weight-stationary K3 (bf16 GEMMs, either stream); fp32
+// GEMMs and 64 channels (the template stack) run the generic tile kernels.
 // mx.heads > 0 runs the MHR mix in K3 (always the generic K3).
 template <class TZ, class TC, int C>
 int trimul_launch(const void* z, const float* mask, const float* lniw, const float* lnib, float eps_in,
@@ -1761,7 +1809,7 @@ int trimul_launch(const void* z, const float* mask, const float* lniw, const flo
                                                                   outgoing);
       (void)grid;
     }
-    else if constexpr (sizeof(TC) == 2 && C == 256 && sizeof(TZ) == 2) {  // (fp32 rows would spill)
+    else if constexpr (sizeof(TC) == 2 && C == 256) {
       const long ntiles = (long)B * Np * (Np / Project256::BP);
       const int nblk = (int)std::min<long>(ntiles, pf::cu_count());
       trimul_project256_kernel<TZ><<<nblk, Project256::NT, 0, s>>>((const TZ*)z, mask, lniw, lnib, eps_in,
@@ -1817,15 +1865,21 @@ int trimul_launch(const void* z, const float* mask, const float* lniw, const flo
                                                                 eps_in, lnow, lnob, eps_out, (const bf16*)wo,
                                                                 (const bf16*)wog, B, N, Np, accumulate);
       (void)grid;
-    } else if constexpr (sizeof(TC) == 2 && C == 256 && sizeof(TZ) == 2) {
+    } else if constexpr (sizeof(TC) == 2 && C == 256) {
       const long ntiles = (long)B * N * ((N + Output256::BP - 1) / Output256::BP);
-      PF_REQUIRE(ntiles < (1L << 31) && (long)Np * Np * Output256::C < (1L << 31), PF_ERR_UNSUPPORTED,
+      const bool fits = ntiles < (1L << 31) && (long)Np * Np * Output256::C < (1L << 31);
+      PF_REQUIRE(fits || sizeof(TZ) == 4, PF_ERR_UNSUPPORTED,
                  "trimul_output: N=%d B=%d (B N ceil(N/64) and 256 Np^2 must stay below 2^31)", N, B);
       const int nblk = (int)std::min<long>(ntiles, pf::cu_count());
-      trimul_output256_kernel<<<nblk, Output256::NT, 0, s>>>((const bf16*)X, (const bf16*)z, (bf16*)out, lniw, lnib,
-                                                             eps_in, lnow, lnob, eps_out, (const bf16*)wo,
-                                                             (const bf16*)wog, B, N, Np, accumulate);
-      (void)grid;
+      if (!fits) {  // an fp32 stream past the persistent kernel's 32-bit plane offsets: the tile kernel
+        if constexpr (sizeof(TZ) == 4)
+          trimul_output_kernel<TZ, TC, C><<<grid, trimul_nt<C>(), 0, s>>>(
+              X, (const TZ*)z, (TZ*)out, lniw, lnib, eps_in, lnow, lnob, eps_out, (const TC*)wo, (const TC*)wog, B, N,
+              Np, accumulate, mx);
+      } else
+        trimul_output256_kernel<TZ><<<nblk, Output256::NT, 0, s>>>((const bf16*)X, (const TZ*)z, (TZ*)out, lniw, lnib,
+                                                                   eps_in, lnow, lnob, eps_out, (const bf16*)wo,
+                                                                   (const bf16*)wog, B, N, Np, accumulate);
     } else
       trimul_output_kernel<TZ, TC, C><<<grid, trimul_nt<C>(), 0, s>>>(X, (const TZ*)z, (TZ*)out, lniw, lnib, eps_in, lnow,
                                                            lnob, eps_out, (const TC*)wo, (const TC*)wog, B, N, Np,

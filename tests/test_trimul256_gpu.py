@@ -1,4 +1,4 @@
-"""GPU: triangle multiplication at 256 channels with bf16 GEMMs and a bf16 stream (reference
+"""GPU: triangle multiplication at 256 channels with bf16 GEMMs on a bf16 or fp32 stream (reference
 ``ops.py:412-473``, ``:645-680`` at the production width of ``configs/stage0.yaml:54-56``).
 
 This regime runs the persistent 256-channel kernels: the weight-streaming projection (K1,
@@ -95,3 +95,27 @@ def test_trimul256_residual_in_place(dev, outgoing):
     err = (got.float() - want).abs().max().item()
     tol = 2.0**-7 * want.abs().max().item()
     assert err <= tol, f"in-place residual: max |diff| {err:.3e} > {tol:.3e}"
+
+
+@pytest.mark.parametrize("outgoing", [True, False], ids=["out", "in"])
+@pytest.mark.parametrize("n,batch", [(5, 1), (64, 2), (130, 1), (200, 1)])
+def test_trimul256_fp32_stream(dev, n, batch, outgoing):
+    """The fp32 stream under bf16 autocast: the same persistent kernels (K1's rows clamped past
+    N, K3 reading its residual rows again), by the bf16 rule against fp64, batch items
+    independent, and the in-place residual equal to z + forward(z) (both fp32: exact)."""
+    m, p = _trimul(dev, outgoing, 120 + n)
+    m = m.float()
+    print(f"[trimul256 fp32 stream] N={n} batch={batch} outgoing={outgoing}", flush=True)
+    z = _z(n, n + 5, batch).to(dev)
+    mask = _mask(n, n + 6, batch, pad=min(6, n // 3)).to(dev)
+    with torch.no_grad():
+        with torch.autocast("cuda", dtype=BF):
+            got = m(z, mask)
+            res = m.forward_residual_(z.clone(), mask)
+            one = m(z[-1:], mask[-1:])
+            eager = R.tri_mul(z, mask, to(p, dev), outgoing)
+        ref = R.tri_mul(z.double(), mask.double(), to(p, dev, torch.float64), outgoing)
+    assert got.dtype == torch.float32 and torch.equal(one, got[-1:])
+    assert torch.equal(res, z + got)
+    print(f"[trimul256 fp32 stream N={n}]",
+          assert_bf16_rule(got.cpu(), eager.float().cpu(), ref.cpu(), f"trimul256 fp32 stream N={n}"), flush=True)  # fmt: skip
