@@ -473,6 +473,14 @@ PF_DEVICE void lds_barrier() {
   __builtin_amdgcn_s_barrier();
 }
 
+// lds_barrier() that also keeps the compiler from moving memory accesses across it, for
+// kernels whose LDS is filled by loads the compiler does not see (buf_load_lds16_async).
+PF_DEVICE void lds_barrier_fenced() {
+  asm volatile("" ::: "memory");
+  lds_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // ---------------------------------------------------------------- 16-value fragments
 // Key order of a 32-key block in flash-attention operands. With S^T = K Q^T on a 32x32
 // MFMA, lane (q, h) (q = lane & 31, h = lane >> 5) holds the logits of query q for keys

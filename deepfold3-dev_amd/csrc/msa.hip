@@ -12,8 +12,9 @@
 //     [N][Kp] x [S D][Kp]^T), gates with sigmoid(to_g(LN(msa))) and projects with out_proj,
 //     stored into or added to the MSA stream.
 //
-// LayerNorms and the thin projections use the row kernels; the contractions use the batched
-// NT GEMM (k zero-padded to its tile).
+// With bf16 operands at the stack's widths the outer product mean is two fused kernels;
+// otherwise LayerNorms and the thin projections use the row kernels and the contractions the
+// batched NT GEMM (k zero-padded to its tile).
 #include <algorithm>
 
 #include "capi.h"
@@ -28,8 +29,15 @@ long pad_k(long k) { return (k + kBgemmK - 1) / kBgemmK * kBgemmK; }
 
 // ------------------------------------------------------------------ outer product mean
 struct OpmWs {
-  size_t xn, ab, at, bt, mt, x, y, act, cnt, total;
+  size_t xn, ab, at, bt, mt, x, y, act, cnt, wf, total;
 };
+
+// The fused outer-product-mean kernels serve bf16 operands at the MSA stack's widths (64 MSA
+// channels, 32 hidden, 128 or 256 pair channels); any other widths and fp32 operands take the
+// batched GEMMs.
+bool opm_fused(int Cm, int CH, int Cz, int cdtype) {
+  return cdtype == PF_BF16 && Cm == 64 && CH == 32 && (Cz == 128 || Cz == 256);
+}
 
 OpmWs opm_layout(int B, int S, int N, int Cm, int CH, int Cz, int cdtype) {
   const size_t es = es_of(cdtype);
@@ -42,6 +50,15 @@ OpmWs opm_layout(int B, int S, int N, int Cm, int CH, int Cz, int cdtype) {
     off += pf::round_up(bytes, 256);
     return at;
   };
+  w = OpmWs{};
+  if (opm_fused(Cm, CH, Cz, cdtype)) {
+    w.at = take((size_t)B * N * CH * Sp * es);
+    w.bt = take((size_t)B * N * CH * Sp * es);
+    w.mt = take((size_t)B * N * Sp * 4);
+    w.wf = take((size_t)Cz * CH * CH * es);
+    w.total = off;
+    return w;
+  }
   w.xn = take(R * Cm * es);
   w.ab = take(R * 2 * CH * es);
   w.at = take((size_t)B * N * CH * Sp * es);
@@ -76,21 +93,24 @@ __global__ __launch_bounds__(256) void opm_pack_kernel(const TC* __restrict__ ab
   Mt[((size_t)b * N + i) * Sp + s] = m;
 }
 
-// Y[b][i N + j][e CH + f] = X[b][i CH + e][j CH + f]; one thread per element of Y.
+// Y[b][i N + j][e CH + f] = X[b][i CH + e][j CH + f]; one thread per 16 bytes of Y (CH is a
+// multiple of 8, so a piece stays inside one row of X).
 template <class TC>
 __global__ __launch_bounds__(256) void opm_reorder_kernel(const TC* __restrict__ X, TC* __restrict__ Y, int B, int N,
                                                           int CH) {
-  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  const long ch2 = (long)CH * CH;
-  if (idx >= (long)B * N * N * ch2) return;
-  const int f = (int)(idx % CH);
-  const int e = (int)((idx / CH) % CH);
-  const long ij = idx / ch2;
-  const int j = (int)(ij % N);
-  const int i = (int)((ij / N) % N);
-  const int b = (int)(ij / ((long)N * N));
+  constexpr int VEC = 16 / sizeof(TC);
+  const long piece = (long)blockIdx.x * 256 + threadIdx.x;
+  const int ch2 = CH * CH;
+  if (piece >= (long)B * N * N * ch2 / VEC) return;
+  const long ij = piece / (ch2 / VEC);
+  const int ef = (int)(piece - ij * (ch2 / VEC)) * VEC;
+  const int e = ef / CH, f = ef - e * CH;
+  const long bi = ij / N;
+  const int j = (int)(ij - bi * N);
+  const int b = (int)(bi / N), i = (int)(bi - (long)b * N);
   const long NC = (long)N * CH;
-  Y[idx] = X[(size_t)b * NC * NC + ((size_t)i * CH + e) * NC + (size_t)j * CH + f];
+  *reinterpret_cast<u32x4*>(Y + piece * VEC) =
+      *reinterpret_cast<const u32x4*>(X + (size_t)b * NC * NC + ((size_t)i * CH + e) * NC + (size_t)j * CH + f);
 }
 
 // out[b,i,j,c] (+)= (act + out_b[c]) / (1e-3 + cnt[b,i,j]).
@@ -130,7 +150,8 @@ int opm_launch(const void* msa, const float* mask, const float* lnw, const float
   const long NC = (long)N * CH;
   if (int e = bgemm_nt(At, Bt, X, (int)NC, (int)NC, Sp, Sp, Sp, NC, NC * Sp, NC * Sp, NC * NC, B, cd, cd, s)) return e;
   const long ny = (long)B * N * N * CH * CH;
-  opm_reorder_kernel<TC><<<(unsigned)((ny + 255) / 256), 256, 0, s>>>(X, Y, B, N, CH);
+  const long npiece = ny / (16 / (long)sizeof(TC));
+  opm_reorder_kernel<TC><<<(unsigned)((npiece + 255) / 256), 256, 0, s>>>(X, Y, B, N, CH);
   if (int e = pf::check_launch("opm_reorder")) return e;
   const long NN = (long)B * N * N;
   if (int e = bgemm_nt(Y, w_out, act, (int)NN, Cz, CH * CH, CH * CH, CH * CH, Cz, 0, 0, 0, 1, cd, PF_F32, s)) return e;
@@ -139,6 +160,344 @@ int opm_launch(const void* msa, const float* mask, const float* lnw, const float
   opm_epilogue_kernel<TZ><<<(unsigned)((NN * Cz + 255) / 256), 256, 0, s>>>(act, b_out, cnt, (TZ*)out, NN, Cz,
                                                                             accumulate);
   return pf::check_launch("opm_epilogue");
+}
+
+
+// ---- fused path (bf16 operands): two launches.
+//
+// opm_project: LayerNorm, both projections and the mask, written sequence-minor for the
+// contraction (At, Bt [b][i 32 + e][Sp], Mt [b][i][Sp]); a block takes 64 sequences of 4
+// residues, a wave the 64 x 64 x 64 product of one residue, whose transposed result goes
+// through the wave's own rows of the LDS tile. Blocks past the tiles lay out_w out in the
+// order in which the contraction kernel's lanes read it (Wf). One pass over the MSA, bound by
+// memory: 16 us at S=512, N=384 bf16, where LayerNorm, row GEMM and pack took 65.
+constexpr int kOpmCH = 32;
+struct OpmProj {
+  static constexpr int C = 64;
+  static constexpr int TS = 64;  // sequences per block
+  static constexpr int TR = 4;   // residues per block, one per wave
+  static constexpr int LD = C + 8;
+};
+
+template <class TM>
+__global__ __launch_bounds__(256) void opm_project_kernel(const TM* __restrict__ msa, const float* __restrict__ mask,
+                                                          const float* __restrict__ lnw, const float* __restrict__ lnb,
+                                                          float eps, const bf16* __restrict__ w_ab,
+                                                          const bf16* __restrict__ w_out, bf16* __restrict__ At,
+                                                          bf16* __restrict__ Bt, float* __restrict__ Mt,
+                                                          bf16* __restrict__ Wf, int B, int S, int N, int Sp, int Cz,
+                                                          int ntile) {
+  using Cfg = OpmProj;
+  constexpr int C = Cfg::C, TS = Cfg::TS, TR = Cfg::TR, LD = Cfg::LD;
+  __shared__ __attribute__((aligned(16))) bf16 xs[TR * TS * LD];
+  __shared__ __attribute__((aligned(16))) float mk[TR * TS];
+  const int tid = threadIdx.x;
+  if ((int)blockIdx.x >= ntile) {
+    // Wf piece (c / 32, step t, lane (hf, c % 32)) = out_w[c][e][8 g ..], 2 t + hf = 32 g + e
+    const int piece = ((int)blockIdx.x - ntile) * 256 + tid;
+    if (blockIdx.y != 0 || piece >= Cz * kOpmCH * kOpmCH / 8) return;
+    const int l = piece & 63, t = (piece >> 6) & 63, cg = piece >> 12;
+    const int p = 2 * t + (l >> 5);
+    const int c = 32 * cg + (l & 31);
+    *reinterpret_cast<u32x4*>(Wf + (size_t)piece * 8) = *reinterpret_cast<const u32x4*>(
+        w_out + ((size_t)c * kOpmCH + (p & 31)) * kOpmCH + 8 * (p >> 5));
+    return;
+  }
+  const int b = blockIdx.y;
+  const int nst = Sp / TS;
+  const int i0 = ((int)blockIdx.x / nst) * TR;
+  const int s0 = ((int)blockIdx.x % nst) * TS;
+  ln_tile_to_lds<TM, bf16, C, TR * TS, 256>(
+      [&](int p) -> const TM* {
+        const int i = i0 + (p >> 6), q = s0 + (p & 63);
+        return (i < N && q < S) ? msa + (((size_t)b * S + q) * N + i) * C : nullptr;
+      },
+      lnw, lnb, eps, xs, LD);
+  {
+    const int i = i0 + (tid & 3), q = s0 + (tid >> 2);
+    mk[(tid & 3) * TS + (tid >> 2)] = (i < N && q < S) ? mask[((size_t)b * S + q) * N + i] : 0.f;
+  }
+  __syncthreads();
+  const int w = wave_id();
+  const int l = lane_id();
+  const int lq = l & 31, hf = l >> 5;
+  const int i = i0 + w;
+  if (i >= N) return;  // no barrier follows
+  bf16* xw = xs + w * TS * LD;
+  const float* mw = mk + w * TS;
+  f32x16 acc[2][2];  // [32 sequences][a | b]
+  zero_acc32(acc);
+#pragma unroll
+  for (int ks = 0; ks < C / 16; ++ks) {
+    bf16x8 wf[2];
+#pragma unroll
+    for (int ab = 0; ab < 2; ++ab)
+      wf[ab] = *reinterpret_cast<const bf16x8*>(w_ab + (size_t)(32 * ab + lq) * C + 16 * ks + 8 * hf);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const bf16x8 xf = *reinterpret_cast<const bf16x8*>(xw + (32 * t + lq) * LD + 16 * ks + 8 * hf);
+#pragma unroll
+      for (int ab = 0; ab < 2; ++ab) acc[t][ab] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, wf[ab], acc[t][ab], 0, 0, 0);
+    }
+  }
+  // acc[t][ab][4 g + e]: hidden channel lq, sequence 32 t + 8 g + 4 hf + e. The wave's rows of
+  // xs are its own: its LDS operations complete in order, no barrier.
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int sq = 32 * t + acc32_row(4 * g);
+      const f32x4 m4 = *reinterpret_cast<const f32x4*>(mw + sq);
+#pragma unroll
+      for (int ab = 0; ab < 2; ++ab) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[t][ab][4 * g + e] * m4[e];
+        store_vec<bf16, 4>(xw + (32 * ab + lq) * LD + sq, v);
+      }
+    }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int it = 0; it < 8; ++it) {
+    const int row = it * 8 + (l >> 3);  // a channels, then b channels
+    bf16* dst = (row < 32 ? At : Bt) + (((size_t)b * N + i) * kOpmCH + (row & 31)) * Sp + s0 + 8 * (l & 7);
+    *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(xw + row * LD + 8 * (l & 7));
+  }
+  Mt[((size_t)b * N + i) * Sp + s0 + l] = mw[l];
+}
+
+// opm_contract: one 8-wave block per tile of 8 x 8 residue pairs. The outer product's 256 x
+// 256 x Sp GEMM (rows (j, f), columns (i, e)) runs on two 64 KB LDS stages of 64-sequence
+// k-tiles filled by direct buffer loads one tile ahead, one barrier per k-tile, each wave 128
+// x 64 of it. Its result, rounded to bf16, is the second operand of the out_w product: it stays
+// in LDS as [pair][piece] (64 x 2 KB, over the two stages) instead of making the N^2 CH^2
+// round trips (store, reorder, load) through memory that bounded the three-launch form. A
+// 32 x 32 accumulator block holds four consecutive f of one e per lane, so the pieces are
+// (f / 8, e): stores and 16-byte fragment reads are conflict-free with the piece index XORed
+// by the pair, and out_w is read in that order (Wf). The 64 x Cz x 1024 product splits the
+// channels over four waves and k over two; the halves meet in an fp32 stage, where the
+// bias, the mask count (each pair's sum over the sequences, formed per tile) and the residual
+// apply. Smaller tiles would re-read out_w (256 KB per tile at Cz = 128) more often. Blocks go
+// to the XCDs so that the 32 tiles an XCD runs at once share 4 row and 8 column strips (3 MB at
+// Sp = 512, inside its L2). Measured at S=512, N=384 bf16: 235 us (195 GFLOP), against 985 us
+// for the batched GEMM, reorder, out_w GEMM, count GEMM and epilogue (245 + 611 + 91 + 41 +
+// 34); bound by the matrix pipe and, per tile, the serial phases around its k loop.
+struct OpmCon {
+  static constexpr int T = 8;               // residues per tile side
+  static constexpr int R = T * kOpmCH;      // 256 operand rows
+  static constexpr int KT = 64;             // sequences per k-tile: 128-byte rows
+  static constexpr int HALF = R * KT * 2;   // one operand's k-tile
+  static constexpr int STAGE = 2 * HALF;
+  static constexpr int NT = 512;
+  static constexpr int STEPS = kOpmCH * kOpmCH / 16;  // 16-wide k-steps of the out_w product
+  static constexpr int GI = 4;              // row strips per XCD group
+};
+
+template <class TZ, int CZ>
+__global__ __launch_bounds__(OpmCon::NT, 1) void opm_contract_kernel(
+    const bf16* __restrict__ At, const bf16* __restrict__ Bt, const float* __restrict__ Mt,
+    const bf16* __restrict__ Wf, const float* __restrict__ bias, TZ* __restrict__ out, int N, int Sp, int nt,
+    int accumulate) {
+  using Cfg = OpmCon;
+  constexpr int NC = CZ / 128;
+  constexpr int SLD = CZ + 4;
+  constexpr int OUT = 2 * 64 * SLD * 4;  // the k halves' fp32 stages, over the operand stages
+  __shared__ __attribute__((aligned(16))) char smem[OUT > 2 * Cfg::STAGE ? OUT : 2 * Cfg::STAGE];
+  __shared__ float cnt[64];
+
+  const int tid = threadIdx.x;
+  const int w = wave_id();
+  const int l = lane_id();
+  const int lq = l & 31, hf = l >> 5;
+  int it, jt;
+  {
+    const int T = nt * nt, x = blockIdx.x & 7;
+    const int seq = x * (T >> 3) + min(x, T & 7) + (int)(blockIdx.x >> 3);
+    const int g = seq / (Cfg::GI * nt);
+    const int rem = seq - g * Cfg::GI * nt;
+    const int gi = min(Cfg::GI, nt - g * Cfg::GI);
+    jt = rem / gi;
+    it = g * Cfg::GI + (rem - jt * gi);
+  }
+  const int b = blockIdx.y;
+  const int i0 = it * Cfg::T, j0 = jt * Cfg::T;
+
+  const int ra = min(Cfg::R, (N - i0) * kOpmCH), rb = min(Cfg::R, (N - j0) * kOpmCH);  // operand rows in range
+  const i32x4_t rsa = buf_rsrc_words(At + ((size_t)b * N + i0) * kOpmCH * Sp, (unsigned)ra * Sp * 2);
+  const i32x4_t rsb = buf_rsrc_words(Bt + ((size_t)b * N + j0) * kOpmCH * Sp, (unsigned)rb * Sp * 2);
+  // Row r's logical 16-byte piece p sits at p ^ ((r >> 1) & 7); rows past N repeat the last one
+  // (their products are not stored).
+  int offa[4], offb[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int row = 8 * (4 * w + q) + (l >> 3);
+    const int lc = (l & 7) ^ ((row >> 1) & 7);
+    offa[q] = min(row, ra - 1) * Sp * 2 + 16 * lc;
+    offb[q] = min(row, rb - 1) * Sp * 2 + 16 * lc;
+  }
+  auto issue = [&](int kt) __attribute__((always_inline)) {
+    char* st = smem + (kt & 1) * Cfg::STAGE;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      buf_load_lds16_async(rsa, st + (4 * w + q) * 1024, offa[q], kt * Cfg::KT * 2);
+      buf_load_lds16_async(rsb, st + Cfg::HALF + (4 * w + q) * 1024, offb[q], kt * Cfg::KT * 2);
+    }
+  };
+  issue(0);
+  {  // mask counts: 8 lanes per pair
+    const int p = tid >> 3, part = tid & 7;
+    const f32x4* mi = reinterpret_cast<const f32x4*>(Mt + ((size_t)b * N + min(i0 + (p >> 3), N - 1)) * Sp);
+    const f32x4* mj = reinterpret_cast<const f32x4*>(Mt + ((size_t)b * N + min(j0 + (p & 7), N - 1)) * Sp);
+    float s = 0.f;
+    for (int q = part; q < Sp / 4; q += 8) {
+      const f32x4 a = mi[q], c = mj[q];
+      s += a[0] * c[0] + a[1] * c[1] + a[2] * c[2] + a[3] * c[3];
+    }
+    s = dpp_sum8(s);
+    if (part == 0) cnt[p] = s;
+  }
+
+  const int jw = w & 1, iw = w >> 1;  // this wave's j residues 4 jw .. and i residues 2 iw ..
+  f32x16 acc[4][2];
+  zero_acc32(acc);
+  const int nk = Sp / Cfg::KT;
+  const int sw = (lq >> 1) & 7;  // swizzle of this lane's rows (the bases are multiples of 16)
+  for (int kt = 0; kt < nk; ++kt) {
+    __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // vmcnt(0): this wave's k-tile kt landed
+    lds_barrier_fenced();
+    if (kt + 1 < nk) issue(kt + 1);
+    const char* sa = smem + (kt & 1) * Cfg::STAGE + (64 * iw + lq) * 128;
+    const char* sb = smem + (kt & 1) * Cfg::STAGE + Cfg::HALF + (128 * jw + lq) * 128;
+#pragma unroll
+    for (int ks = 0; ks < Cfg::KT / 16; ++ks) {
+      const int po = 16 * ((2 * ks + hf) ^ sw);
+      bf16x8 fa[2], fb[4];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) fa[q] = *reinterpret_cast<const bf16x8*>(sa + q * 32 * 128 + po);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) fb[q] = *reinterpret_cast<const bf16x8*>(sb + q * 32 * 128 + po);
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+        for (int ii = 0; ii < 2; ++ii)
+          acc[jj][ii] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[jj], fa[ii], acc[jj][ii], 0, 0, 0);
+    }
+  }
+  // ---- X -> LDS [pair = 8 i + j][piece 32 g + e]: lane (e = lq) holds f = 8 g + 4 hf + 0..3
+  const int cg = w & 3, kh = w >> 2;  // channels 32 cg .. (+ 128), k-steps 32 kh ..
+  constexpr int HS = Cfg::STEPS / 2;
+  constexpr int GRP = NC == 1 ? 8 : 4;  // fragments of out_w in flight
+  const bf16x8* wp = reinterpret_cast<const bf16x8*>(Wf) + ((size_t)cg * Cfg::STEPS + kh * HS) * 64 + l;
+  bf16x8 wf[GRP][NC];
+  auto load_w = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < GRP; ++t)
+#pragma unroll
+      for (int n = 0; n < NC; ++n) wf[t][n] = wp[((size_t)n * 4 * Cfg::STEPS + t0 + t) * 64];
+  };
+  load_w(0);
+  lds_barrier_fenced();  // every wave is done with the operand stages
+#pragma unroll
+  for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+    for (int ii = 0; ii < 2; ++ii) {
+      const int pair = 8 * (2 * iw + ii) + 4 * jw + jj;
+      char* xr = smem + pair * 2048 + 8 * hf;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[jj][ii][4 * g + e];
+        store_vec<bf16, 4>(reinterpret_cast<bf16*>(xr + 16 * ((32 * g + lq) ^ (pair & 15))), v);
+      }
+    }
+  lds_barrier_fenced();
+  f32x16 acc2[NC][2];  // [channels 128 n + 32 cg ..][pairs 32 t ..]
+  zero_acc32(acc2);
+#pragma unroll 1
+  for (int t0 = 0; t0 < HS; t0 += GRP) {
+    bf16x8 wc[GRP][NC];
+#pragma unroll
+    for (int t = 0; t < GRP; ++t)
+#pragma unroll
+      for (int n = 0; n < NC; ++n) wc[t][n] = wf[t][n];
+    if (t0 + GRP < HS) load_w(t0 + GRP);
+#pragma unroll
+    for (int t = 0; t < GRP; ++t) {
+      const int p = 2 * (kh * HS + t0 + t) + hf;
+      bf16x8 xf[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        xf[q] = *reinterpret_cast<const bf16x8*>(smem + (32 * q + lq) * 2048 + 16 * (p ^ (lq & 15)));
+#pragma unroll
+      for (int n = 0; n < NC; ++n)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          acc2[n][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wc[t][n], xf[q], acc2[n][q], 0, 0, 0);
+    }
+  }
+  lds_barrier_fenced();  // every wave is done with X
+  float* st = reinterpret_cast<float*>(smem) + kh * 64 * SLD;
+#pragma unroll
+  for (int n = 0; n < NC; ++n)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4*>(st + (32 * q + lq) * SLD + 128 * n + 32 * cg + acc32_row(4 * g)) =
+            f32x4{acc2[n][q][4 * g], acc2[n][q][4 * g + 1], acc2[n][q][4 * g + 2], acc2[n][q][4 * g + 3]};
+  lds_barrier_fenced();
+  constexpr int VEC = 16 / sizeof(TZ);
+  constexpr int PPR = CZ / VEC;
+  const float* s0 = reinterpret_cast<const float*>(smem);
+#pragma unroll
+  for (int k = 0; k < 64 * PPR / Cfg::NT; ++k) {
+    const int idx = k * Cfg::NT + tid;
+    const int pair = idx / PPR, c0 = (idx % PPR) * VEC;
+    const int i = i0 + (pair >> 3), j = j0 + (pair & 7);
+    if (i >= N || j >= N) continue;
+    TZ* dst = out + (((size_t)b * N + i) * N + j) * CZ + c0;
+    float v[VEC], r[VEC];
+    const float den = 1e-3f + cnt[pair];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)
+      v[e] = (s0[pair * SLD + c0 + e] + s0[(64 + pair) * SLD + c0 + e] + bias[c0 + e]) / den;
+    if (accumulate) {
+      load16<TZ>(dst, r);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[e] += r[e];
+    }
+    store_vec<TZ, VEC>(dst, v);
+  }
+}
+
+template <class TM, class TZ>
+int opm_fused_launch(const void* msa, const float* mask, const float* lnw, const float* lnb, float eps,
+                     const void* w_ab, const void* w_out, const float* b_out, int B, int S, int N, int Cz, void* out,
+                     int accumulate, void* ws, hipStream_t s) {
+  const OpmWs L = opm_layout(B, S, N, OpmProj::C, kOpmCH, Cz, PF_BF16);
+  const int Sp = (int)pad_k(S);
+  char* base = reinterpret_cast<char*>(ws);
+  bf16* At = reinterpret_cast<bf16*>(base + L.at);
+  bf16* Bt = reinterpret_cast<bf16*>(base + L.bt);
+  float* Mt = reinterpret_cast<float*>(base + L.mt);
+  bf16* Wf = reinterpret_cast<bf16*>(base + L.wf);
+  const int ntile = (N + OpmProj::TR - 1) / OpmProj::TR * (Sp / OpmProj::TS);
+  const int nw = (Cz * kOpmCH * kOpmCH / 8 + 255) / 256;
+  opm_project_kernel<TM><<<dim3((unsigned)(ntile + nw), (unsigned)B), 256, 0, s>>>(
+      (const TM*)msa, mask, lnw, lnb, eps, (const bf16*)w_ab, (const bf16*)w_out, At, Bt, Mt, Wf, B, S, N, Sp, Cz,
+      ntile);
+  if (int e = pf::check_launch("opm_project")) return e;
+  const int nt = (N + OpmCon::T - 1) / OpmCon::T;
+  const dim3 grid((unsigned)(nt * nt), (unsigned)B);
+  if (Cz == 128)
+    opm_contract_kernel<TZ, 128><<<grid, OpmCon::NT, 0, s>>>(At, Bt, Mt, Wf, b_out, (TZ*)out, N, Sp, nt, accumulate);
+  else
+    opm_contract_kernel<TZ, 256><<<grid, OpmCon::NT, 0, s>>>(At, Bt, Mt, Wf, b_out, (TZ*)out, N, Sp, nt, accumulate);
+  return pf::check_launch("opm_contract");
 }
 
 // ------------------------------------------------------------------ MSA pair-weighted averaging
@@ -309,6 +668,17 @@ int pf_outer_product_mean_fwd(const void* msa, const float* msa_mask, const floa
   if (mdtype == PF_F32 && cdtype == PF_F32)
     return opm_launch<float, float, float>(msa, msa_mask, ln_w, ln_b, eps, w_ab, w_out, b_out, B, S, N, Cm, CH, Cz,
                                            out, accumulate, workspace, s);
+  // grid.y is the batch; the staged operands are addressed with 32-bit byte offsets per tile
+  if (opm_fused(Cm, CH, Cz, cdtype)) {
+    PF_REQUIRE(B < 65536 && (long)OpmCon::R * pad_k(S) * 2 < (1L << 31) &&
+                   (long)((N + 3) / 4) * (pad_k(S) / 64) < (1L << 30),
+               PF_ERR_UNSUPPORTED, "pf_outer_product_mean_fwd: B=%d S=%d N=%d", B, S, N);
+    if (mdtype == PF_F32)
+      return opm_fused_launch<float, float>(msa, msa_mask, ln_w, ln_b, eps, w_ab, w_out, b_out, B, S, N, Cz, out,
+                                            accumulate, workspace, s);
+    return opm_fused_launch<bf16, bf16>(msa, msa_mask, ln_w, ln_b, eps, w_ab, w_out, b_out, B, S, N, Cz, out,
+                                        accumulate, workspace, s);
+  }
   if (mdtype == PF_F32)
     return opm_launch<float, bf16, float>(msa, msa_mask, ln_w, ln_b, eps, w_ab, w_out, b_out, B, S, N, Cm, CH, Cz, out,
                                           accumulate, workspace, s);
