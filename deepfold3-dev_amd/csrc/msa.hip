@@ -33,10 +33,11 @@ struct OpmWs {
 };
 
 // The fused outer-product-mean kernels serve bf16 operands at the MSA stack's widths (64 MSA
-// channels, 32 hidden, 128 or 256 pair channels); any other widths and fp32 operands take the
-// batched GEMMs.
-bool opm_fused(int Cm, int CH, int Cz, int cdtype) {
-  return cdtype == PF_BF16 && Cm == 64 && CH == 32 && (Cz == 128 || Cz == 256);
+// channels, 32 hidden, 128 or 256 pair channels) on 16-byte aligned tensors, within their grid
+// and 32-bit offsets; anything else takes the batched GEMMs. The workspace holds either.
+bool opm_fused(int B, int S, int N, int Cm, int CH, int Cz, int cdtype) {
+  return cdtype == PF_BF16 && Cm == 64 && CH == 32 && (Cz == 128 || Cz == 256) && B < 65536 && S < (1 << 20) &&
+         (long)(N + 3) / 4 * (pad_k(S) / kBgemmK) < (1L << 30);
 }
 
 OpmWs opm_layout(int B, int S, int N, int Cm, int CH, int Cz, int cdtype) {
@@ -50,15 +51,7 @@ OpmWs opm_layout(int B, int S, int N, int Cm, int CH, int Cz, int cdtype) {
     off += pf::round_up(bytes, 256);
     return at;
   };
-  w = OpmWs{};
-  if (opm_fused(Cm, CH, Cz, cdtype)) {
-    w.at = take((size_t)B * N * CH * Sp * es);
-    w.bt = take((size_t)B * N * CH * Sp * es);
-    w.mt = take((size_t)B * N * Sp * 4);
-    w.wf = take((size_t)Cz * CH * CH * es);
-    w.total = off;
-    return w;
-  }
+  w.wf = take((size_t)Cz * CH * CH * es);  // fused path: at, bt, mt and this
   w.xn = take(R * Cm * es);
   w.ab = take(R * 2 * CH * es);
   w.at = take((size_t)B * N * CH * Sp * es);
@@ -505,6 +498,16 @@ struct PavWs {
   size_t pn, lg, cm, w, xm, vg, vt, va, og, total;
 };
 
+// The fused pair-weighted averaging serves bf16 operands at the MSA stack's widths (64 MSA
+// channels in 8 heads; 64, 128 or 256 pair channels) on 16-byte aligned tensors while a
+// query's logits of all heads fit the LDS (4096 keys: 128 KB); anything else takes the
+// batched GEMMs. The workspace holds either.
+constexpr int kPavMaxKeys = 4096;
+bool pav_fused(int B, int S, int N, int Cm, int Cz, int H, int cdtype) {
+  return cdtype == PF_BF16 && Cm == 64 && H == 8 && (Cz == 64 || Cz == 128 || Cz == 256) && N <= kPavMaxKeys &&
+         B < 65536 && S < (1 << 24);
+}
+
 PavWs pav_layout(int B, int S, int N, int Cm, int Cz, int H, int cdtype) {
   const size_t es = es_of(cdtype);
   const size_t Kp = pad_k(N);
@@ -520,10 +523,10 @@ PavWs pav_layout(int B, int S, int N, int Cm, int Cz, int H, int cdtype) {
   w.pn = take((size_t)B * N * N * Cz * es);
   w.lg = take((size_t)B * N * N * 16 * 4);
   w.cm = take((size_t)B * N * 4);
-  w.w = take((size_t)B * H * N * Kp * es);
+  w.w = take((size_t)B * H * Kp * Kp * es);  // N rows; the fused path's query tiles reach Kp
   w.xm = take(R * Cm * es);
   w.vg = take(R * 2 * Cm * es);
-  w.vt = take((size_t)B * H * S * D * Kp * es);
+  w.vt = take((size_t)B * H * ((S + 7) / 8 * 8) * D * Kp * es);  // S sequences; the fused path's tiles are of 8
   w.va = take((size_t)B * H * N * S * D * es);
   w.og = take(R * Cm * es);
   w.total = off;
@@ -638,6 +641,441 @@ int pav_launch(const void* msa, const float* mask, const void* pair, const float
   return rowgemm_launch<TC, TM, EPI_STORE>(og, w_out, nullptr, 0, out, R, Cm, Cm, s);
 }
 
+// ---- fused path (bf16 operands): three launches, with the two operands of the averaging
+// product written in the order in which its lanes read them (1 KB fragments: 32 rows x 16
+// keys, lane (key half, row), 8 keys each), so that product needs no LDS tiles.
+//
+// pav_values: LayerNorm, the value projection and its transpose, a wave per (sequence, 64
+// residues); fragment rows are (s mod 4, d). Blocks past the tiles form the column mask.
+// pav_weights: a block per query normalises its pair row, forms the 8 heads' logits on
+// MFMAs (LDS, fp32) and writes their softmax; keys N .. Kp-1 get weight zero.
+// pav_average: a block per 64 queries x 8 sequences, a wave per head: the 64 x 64 x Kp
+// product from fragments four k-steps ahead, its result (rounded to bf16) to LDS; then a
+// wave per sequence recomputes LN(msa) and the gate for its 64 positions, applies it and
+// projects, 16-byte stores (and the residual) through an fp32 stage.
+// One pass over the pair and two over the MSA; the gate is recomputed because storing and
+// reading it would be a third and fourth. S=512, N=384 bf16: 17 + 14 + 45 us (the last bound by
+// fragment loads: 1 KB per lane-step from L2, two blocks' worth of tail), where LayerNorms, row
+// GEMMs, column mask, softmax, value transpose, batched GEMM, gate and projection took 530.
+struct Pav {
+  static constexpr int C = 64, H = 8, D = 8;
+  static constexpr int LD = C + 8;
+  static constexpr int TS = 8, TQ = 64;  // pav_average tile
+  static constexpr int SLD = C + 4;      // fp32 stage rows
+};
+
+template <class TM>
+__global__ __launch_bounds__(256) void pav_values_kernel(const TM* __restrict__ msa, const float* __restrict__ mask,
+                                                         const float* __restrict__ lnw, const float* __restrict__ lnb,
+                                                         float eps, const bf16* __restrict__ w_v,
+                                                         bf16* __restrict__ Vf, float* __restrict__ cm, int S, int N,
+                                                         int Kp, int ntile) {
+  constexpr int C = Pav::C, LD = Pav::LD;
+  __shared__ __attribute__((aligned(16))) bf16 xs[256 * LD];
+  const int tid = threadIdx.x;
+  const int b = blockIdx.y;
+  const int w = wave_id();
+  const int l = lane_id();
+  if ((int)blockIdx.x >= ntile) {  // colmask[b][k]: 64 residues, the sequences split over the waves
+    const int k = ((int)blockIdx.x - ntile) * 64 + l;
+    const float* mb = mask + (size_t)b * S * N + min(k, N - 1);
+    float m = -INFINITY;
+#pragma unroll 4
+    for (int q = w; q < S; q += 4) m = fmaxf(m, mb[(size_t)q * N]);
+    float* red = reinterpret_cast<float*>(xs);
+    red[tid] = m;
+    __syncthreads();
+    if (w == 0 && k < N) cm[(size_t)b * N + k] = fmaxf(fmaxf(red[l], red[64 + l]), fmaxf(red[128 + l], red[192 + l]));
+    return;
+  }
+  const int nit = Kp / 64;
+  const int s0 = ((int)blockIdx.x / nit) * 4;
+  const int i0 = ((int)blockIdx.x % nit) * 64;
+  ln_tile_to_lds<TM, bf16, C, 256, 256>(
+      [&](int p) -> const TM* {
+        const int q = s0 + (p >> 6), i = i0 + (p & 63);
+        return (q < S && i < N) ? msa + (((size_t)b * S + q) * N + i) * C : nullptr;
+      },
+      lnw, lnb, eps, xs, LD);
+  __syncthreads();
+  const int sq = s0 + w;
+  if (sq >= S) return;  // no barrier follows
+  const int lq = l & 31, hf = l >> 5;
+  bf16* xw = xs + w * 64 * LD;
+  f32x16 acc[2][2];  // [32 residues][32 channels]
+  zero_acc32(acc);
+#pragma unroll
+  for (int ks = 0; ks < C / 16; ++ks) {
+    bf16x8 wf[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+      wf[n] = *reinterpret_cast<const bf16x8*>(w_v + (size_t)(32 * n + lq) * C + 16 * ks + 8 * hf);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const bf16x8 xf = *reinterpret_cast<const bf16x8*>(xw + (32 * t + lq) * LD + 16 * ks + 8 * hf);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) acc[t][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, wf[n], acc[t][n], 0, 0, 0);
+    }
+  }
+  // acc[t][n][4 g + e]: channel 32 n + lq, residue 32 t + 8 g + 4 hf + e -> the wave's own rows
+  // of xs as [channel][residue]
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[t][n][4 * g + e];
+        store_vec<bf16, 4>(xw + (32 * n + lq) * LD + 32 * t + acc32_row(4 * g), v);
+      }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int d = l & 7, k8 = l >> 3;
+  const int SG = (S + 7) / 8 * 2, KB = Kp / 16;
+#pragma unroll
+  for (int h = 0; h < Pav::H; ++h) {
+    const size_t frag = (((size_t)b * Pav::H + h) * SG + (sq >> 2)) * KB + (i0 >> 4) + (k8 >> 1);
+    *reinterpret_cast<u32x4*>(Vf + frag * 512 + ((k8 & 1) * 32 + (sq & 3) * 8 + d) * 8) =
+        *reinterpret_cast<const u32x4*>(xw + (h * Pav::D + d) * LD + 8 * k8);
+  }
+}
+
+template <class TM, int CZ>
+__global__ __launch_bounds__(512) void pav_weights_kernel(const TM* __restrict__ pair, const float* __restrict__ lnw,
+                                                          const float* __restrict__ lnb, float eps,
+                                                          const bf16* __restrict__ w_lg, const float* __restrict__ cm,
+                                                          bf16* __restrict__ Wf, int N, int Kp) {
+  constexpr int KS = CZ / 32;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  float* lg = reinterpret_cast<float*>(smem);  // [head][Kp + 4]
+  const int LDL = Kp + 4;
+  __shared__ float lnp[2 * CZ];
+  const int w = wave_id();
+  const int l = lane_id();
+  const int r = l & 15, kq = (l >> 4) * 8;
+  const int q = blockIdx.x, b = blockIdx.y;
+  for (int i = threadIdx.x; i < CZ; i += 512) {
+    lnp[i] = lnw[i];
+    lnp[CZ + i] = lnb[i];
+  }
+  bf16x8 wf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) wf[ks] = *reinterpret_cast<const bf16x8*>(w_lg + (size_t)r * CZ + 32 * ks + kq);
+  __syncthreads();
+  const TM* row0 = pair + ((size_t)b * N + q) * N * CZ;
+  // 16 keys per wave and step: lane (r, l >> 4) holds channels 32 ks + kq .. of key r
+  for (int k0 = 16 * w; k0 < Kp; k0 += 128) {
+    const TM* src = row0 + (size_t)min(k0 + r, N - 1) * CZ + kq;  // keys past N are masked below
+    float v[KS][8];
+    float s = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      if constexpr (sizeof(TM) == 2) {
+        load16<TM>(src + 32 * ks, v[ks]);
+      } else {
+        float a[4], c[4];
+        load16<TM>(src + 32 * ks, a);
+        load16<TM>(src + 32 * ks + 4, c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[ks][e] = a[e], v[ks][4 + e] = c[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s += v[ks][e];
+    }
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    const float mean = s * (1.0f / CZ);
+    float qs = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float dv = v[ks][e] - mean;
+        qs += dv * dv;
+      }
+    qs += __shfl_xor(qs, 16, 64);
+    qs += __shfl_xor(qs, 32, 64);
+    const float rstd = rsqrtf(qs * (1.0f / CZ) + eps);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const float* pw = lnp + 32 * ks + kq;
+      bf16x8 xf;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xf[e] = (bf16)((v[ks][e] - mean) * rstd * pw[e] + pw[CZ + e]);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, wf[ks], acc, 0, 0, 0);
+    }
+    // acc[e]: head r, key k0 + 4 (l >> 4) + e
+    if (r < Pav::H) *reinterpret_cast<f32x4*>(lg + r * LDL + k0 + 4 * (l >> 4)) = acc;
+  }
+  __syncthreads();
+  // softmax of head w over the keys; the wave's own LDS row from here on
+  float* lw = lg + w * LDL;
+  const float* cb = cm + (size_t)b * N;
+  float mx = -INFINITY;
+  for (int k = l; k < N; k += 64) {
+    const float x = lw[k] + 1e9f * (cb[k] - 1.0f);
+    lw[k] = x;
+    mx = fmaxf(mx, x);
+  }
+  mx = group_max<64>(mx);
+  float sum = 0.f;
+  for (int k = l; k < Kp; k += 64) {
+    const float e = k < N ? expf(lw[k] - mx) : 0.f;
+    lw[k] = e;
+    sum += e;
+  }
+  const float inv = 1.0f / group_sum<64>(sum);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int KB = Kp / 16;
+  bf16* dst = Wf + ((((size_t)b * Pav::H + w) * (Kp / 32) + (q >> 5)) * KB) * 512 + (q & 31) * 8;
+  for (int k8 = l; k8 < Kp / 8; k8 += 64) {
+    const f32x4 a = *reinterpret_cast<const f32x4*>(lw + 8 * k8), c = *reinterpret_cast<const f32x4*>(lw + 8 * k8 + 4);
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = a[e] * inv, v[4 + e] = c[e] * inv;
+    store_vec<bf16, 8>(dst + (size_t)(k8 >> 1) * 512 + (k8 & 1) * 256, v);
+  }
+}
+
+template <class TM>
+__global__ __launch_bounds__(512, 1) void pav_average_kernel(
+    const bf16* __restrict__ Wf, const bf16* __restrict__ Vf, const TM* __restrict__ msa,
+    const float* __restrict__ lnw, const float* __restrict__ lnb, float eps, const bf16* __restrict__ w_g,
+    const bf16* __restrict__ w_out, TM* __restrict__ out, int S, int N, int Kp, int nq, int accumulate) {
+  constexpr int C = Pav::C, LD = Pav::LD, SLD = Pav::SLD;
+  __shared__ __attribute__((aligned(16))) bf16 og[Pav::TS * Pav::TQ * LD];  // [sequence][query][channel]
+  __shared__ __attribute__((aligned(16))) bf16 xs[8][32 * LD];             // per wave: x, then the fp32 stage
+  static_assert(32 * SLD * 4 <= 2 * 32 * LD * 2, "the stage takes two halves of 16 rows");
+  const int w = wave_id();
+  const int l = lane_id();
+  const int lq = l & 31, hf = l >> 5;
+  // XCD x takes consecutive tiles, the query tiles of one sequence group in a row
+  const int T = gridDim.x, x8 = blockIdx.x & 7;
+  const int seq = x8 * (T >> 3) + min(x8, T & 7) + (int)(blockIdx.x >> 3);
+  const int s0 = (seq / nq) * Pav::TS, q0 = (seq % nq) * Pav::TQ;
+  const int b = blockIdx.y;
+  const int SG = (S + 7) / 8 * 2, KB = Kp / 16;
+
+  // ---- head w: va^T[(s, d)][q] = sum_k V W
+  const bf16x8* vp = reinterpret_cast<const bf16x8*>(Vf) + (((size_t)b * Pav::H + w) * SG + (s0 >> 2)) * KB * 64 + l;
+  const bf16x8* wp = reinterpret_cast<const bf16x8*>(Wf) +
+                     (((size_t)b * Pav::H + w) * (Kp / 32) + (q0 >> 5)) * KB * 64 + l;
+  f32x16 acc[2][2];  // [4 sequences][32 queries]
+  zero_acc32(acc);
+  constexpr int G = 4;  // k-steps per group; Kp is a multiple of 64
+  bf16x8 fv[G][2], fw[G][2];
+  auto load = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < G; ++t)
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        fv[t][n] = vp[((size_t)n * KB + t0 + t) * 64];
+        fw[t][n] = wp[((size_t)n * KB + t0 + t) * 64];
+      }
+  };
+  load(0);
+#pragma unroll 1
+  for (int t0 = 0; t0 < KB; t0 += G) {
+    bf16x8 cv[G][2], cw[G][2];
+#pragma unroll
+    for (int t = 0; t < G; ++t)
+#pragma unroll
+      for (int n = 0; n < 2; ++n) cv[t][n] = fv[t][n], cw[t][n] = fw[t][n];
+    if (t0 + G < KB) load(t0 + G);
+#pragma unroll
+    for (int t = 0; t < G; ++t)
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+          acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cv[t][m], cw[t][n], acc[m][n], 0, 0, 0);
+  }
+  // acc[m][n][4 g + e]: sequence 4 m + g, channel 8 w + 4 hf + e, query 32 n + lq
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[m][n][4 * g + e];
+        store_vec<bf16, 4>(og + ((4 * m + g) * Pav::TQ + 32 * n + lq) * LD + Pav::D * w + 4 * hf, v);
+      }
+  __syncthreads();
+
+  // ---- sequence w: gate and output projection of 64 positions, 32 at a time
+  const int sq = s0 + w;
+  if (sq >= S) return;  // no barrier follows
+  bf16* xw = xs[w];
+  float* st = reinterpret_cast<float*>(xs[w]);
+  constexpr int VEC = 16 / sizeof(TM);
+  constexpr int LPR = C / VEC;    // lanes per position
+  constexpr int PPI = 64 / LPR;   // positions per wave-wide access
+  const int sub = (l % LPR) * VEC;
+  float lw[VEC], lb[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) lw[e] = lnw[sub + e], lb[e] = lnb[sub + e];
+  const size_t base = (((size_t)b * S + sq) * N) * C;
+#pragma unroll 1
+  for (int n = 0; n < 2; ++n) {
+    const int qn = q0 + 32 * n;
+    if (qn >= N) break;
+    // LN(msa) of 32 positions -> xw (positions past N read the last one, unused)
+#pragma unroll
+    for (int it = 0; it < 32 / PPI; ++it) {
+      const int p = it * PPI + l / LPR;
+      float v[VEC];
+      load16<TM>(msa + base + (size_t)min(qn + p, N - 1) * C + sub, v);
+      float s = 0.f;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) s += v[e];
+      const float mean = (LPR == 8 ? dpp_sum8(s) : dpp_sum16(s)) * (1.0f / C);
+      float qs = 0.f;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        const float dv = v[e] - mean;
+        qs += dv * dv;
+      }
+      const float rstd = rsqrtf((LPR == 8 ? dpp_sum8(qs) : dpp_sum16(qs)) * (1.0f / C) + eps);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[e] = (v[e] - mean) * rstd * lw[e] + lb[e];
+      store_vec<bf16, VEC>(xw + p * LD + sub, v);
+    }
+    bf16* ow = og + (w * Pav::TQ + 32 * n) * LD;
+    f32x16 ag[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) ag[m][e] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < C / 16; ++ks) {
+      const bf16x8 xf = *reinterpret_cast<const bf16x8*>(xw + lq * LD + 16 * ks + 8 * hf);
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const bf16x8 gf = *reinterpret_cast<const bf16x8*>(w_g + (size_t)(32 * m + lq) * C + 16 * ks + 8 * hf);
+        ag[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gf, xf, ag[m], 0, 0, 0);
+      }
+    }
+    // gate: channels 32 m + 8 g + 4 hf + 0..3 of position lq, in place
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        bf16* o = ow + lq * LD + 32 * m + acc32_row(4 * g);
+        const bf16x4 a = *reinterpret_cast<const bf16x4*>(o);
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = (float)a[e] * sigmoidf_(ag[m][4 * g + e]);
+        store_vec<bf16, 4>(o, v);
+      }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    f32x16 ao[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) ao[m][e] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < C / 16; ++ks) {
+      const bf16x8 of = *reinterpret_cast<const bf16x8*>(ow + lq * LD + 16 * ks + 8 * hf);
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const bf16x8 gf = *reinterpret_cast<const bf16x8*>(w_out + (size_t)(32 * m + lq) * C + 16 * ks + 8 * hf);
+        ao[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gf, of, ao[m], 0, 0, 0);
+      }
+    }
+    // fp32 stage [16 positions][64], twice
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // reads of x or the first half before the stores
+      __builtin_amdgcn_wave_barrier();
+      if ((lq >> 4) == half) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<f32x4*>(st + (lq & 15) * SLD + 32 * m + acc32_row(4 * g)) =
+                f32x4{ao[m][4 * g], ao[m][4 * g + 1], ao[m][4 * g + 2], ao[m][4 * g + 3]};
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int it = 0; it < 16 / PPI; ++it) {
+        const int p = it * PPI + l / LPR;
+        const int pos = qn + 16 * half + p;
+        if (pos >= N) continue;
+        TM* dst = out + base + (size_t)pos * C + sub;
+        float v[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v[e] = st[p * SLD + sub + e];
+        if (accumulate) {
+          float rv[VEC];
+          load16<TM>(dst, rv);
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) v[e] += rv[e];
+        }
+        store_vec<TM, VEC>(dst, v);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the stage is read before x is rewritten
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+template <class TM, int CZ>
+int pav_weights_launch(const void* pair, const float* plnw, const float* plnb, float peps, const void* w_lg,
+                       const float* cm, bf16* Wf, int B, int N, int Kp, hipStream_t s) {
+  const int lds = Pav::H * (Kp + 4) * 4;
+  const void* fn = (const void*)pav_weights_kernel<TM, CZ>;
+  const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  PF_REQUIRE(e == hipSuccess, PF_ERR_LAUNCH, "pav_weights: cannot reserve %d bytes of LDS: %s", lds,
+             hipGetErrorString(e));
+  pav_weights_kernel<TM, CZ><<<dim3((unsigned)N, (unsigned)B), 512, lds, s>>>((const TM*)pair, plnw, plnb, peps,
+                                                                             (const bf16*)w_lg, cm, Wf, N, Kp);
+  return pf::check_launch("pav_weights");
+}
+
+template <class TM>
+int pav_fused_launch(const void* msa, const float* mask, const void* pair, const float* lnw, const float* lnb,
+                     float eps, const float* plnw, const float* plnb, float peps, const void* w_lg, const void* w_vg,
+                     const void* w_out, int B, int S, int N, int Cz, void* out, int accumulate, void* ws,
+                     hipStream_t s) {
+  const PavWs L = pav_layout(B, S, N, Pav::C, Cz, Pav::H, PF_BF16);
+  const int Kp = (int)pad_k(N);
+  char* base = reinterpret_cast<char*>(ws);
+  float* cm = reinterpret_cast<float*>(base + L.cm);
+  bf16* Wf = reinterpret_cast<bf16*>(base + L.w);
+  bf16* Vf = reinterpret_cast<bf16*>(base + L.vt);
+  const int ntile = (S + 3) / 4 * (Kp / 64);
+  pav_values_kernel<TM><<<dim3((unsigned)(ntile + Kp / 64), (unsigned)B), 256, 0, s>>>(
+      (const TM*)msa, mask, lnw, lnb, eps, (const bf16*)w_vg, Vf, cm, S, N, Kp, ntile);
+  if (int e = pf::check_launch("pav_values")) return e;
+  int e;
+  if (Cz == 64)
+    e = pav_weights_launch<TM, 64>(pair, plnw, plnb, peps, w_lg, cm, Wf, B, N, Kp, s);
+  else if (Cz == 128)
+    e = pav_weights_launch<TM, 128>(pair, plnw, plnb, peps, w_lg, cm, Wf, B, N, Kp, s);
+  else
+    e = pav_weights_launch<TM, 256>(pair, plnw, plnb, peps, w_lg, cm, Wf, B, N, Kp, s);
+  if (e) return e;
+  const int nq = (N + Pav::TQ - 1) / Pav::TQ;
+  const unsigned tiles = (unsigned)((S + Pav::TS - 1) / Pav::TS * nq);
+  pav_average_kernel<TM><<<dim3(tiles, (unsigned)B), 512, 0, s>>>(
+      Wf, Vf, (const TM*)msa, lnw, lnb, eps, (const bf16*)w_vg + Pav::C * Pav::C, (const bf16*)w_out, (TM*)out, S, N,
+      Kp, nq, accumulate);
+  return pf::check_launch("pav_average");
+}
+
 bool dt_ok(int d) { return d == PF_F32 || d == PF_BF16; }
 
 }  // namespace
@@ -668,11 +1106,8 @@ int pf_outer_product_mean_fwd(const void* msa, const float* msa_mask, const floa
   if (mdtype == PF_F32 && cdtype == PF_F32)
     return opm_launch<float, float, float>(msa, msa_mask, ln_w, ln_b, eps, w_ab, w_out, b_out, B, S, N, Cm, CH, Cz,
                                            out, accumulate, workspace, s);
-  // grid.y is the batch; the staged operands are addressed with 32-bit byte offsets per tile
-  if (opm_fused(Cm, CH, Cz, cdtype)) {
-    PF_REQUIRE(B < 65536 && (long)OpmCon::R * pad_k(S) * 2 < (1L << 31) &&
-                   (long)((N + 3) / 4) * (pad_k(S) / 64) < (1L << 30),
-               PF_ERR_UNSUPPORTED, "pf_outer_product_mean_fwd: B=%d S=%d N=%d", B, S, N);
+  if (opm_fused(B, S, N, Cm, CH, Cz, cdtype) && pf::aligned16(msa) && pf::aligned16(out) && pf::aligned16(w_ab) &&
+      pf::aligned16(w_out) && pf::aligned16(workspace)) {
     if (mdtype == PF_F32)
       return opm_fused_launch<float, float>(msa, msa_mask, ln_w, ln_b, eps, w_ab, w_out, b_out, B, S, N, Cz, out,
                                             accumulate, workspace, s);
@@ -710,6 +1145,14 @@ int pf_msa_pair_avg_fwd(const void* msa, const float* msa_mask, const void* pair
   if (mdtype == PF_F32 && cdtype == PF_F32)
     return pav_launch<float, float>(msa, msa_mask, pair, ln_w, ln_b, eps, pair_ln_w, pair_ln_b, pair_eps, w_logits,
                                     w_vg, w_out, B, S, N, Cm, Cz, H, out, accumulate, workspace, s);
+  if (pav_fused(B, S, N, Cm, Cz, H, cdtype) && pf::aligned16(msa) && pf::aligned16(pair) && pf::aligned16(out) &&
+      pf::aligned16(w_logits) && pf::aligned16(w_vg) && pf::aligned16(w_out) && pf::aligned16(workspace)) {
+    if (mdtype == PF_F32)
+      return pav_fused_launch<float>(msa, msa_mask, pair, ln_w, ln_b, eps, pair_ln_w, pair_ln_b, pair_eps, w_logits,
+                                     w_vg, w_out, B, S, N, Cz, out, accumulate, workspace, s);
+    return pav_fused_launch<bf16>(msa, msa_mask, pair, ln_w, ln_b, eps, pair_ln_w, pair_ln_b, pair_eps, w_logits,
+                                  w_vg, w_out, B, S, N, Cz, out, accumulate, workspace, s);
+  }
   if (mdtype == PF_F32)
     return pav_launch<float, bf16>(msa, msa_mask, pair, ln_w, ln_b, eps, pair_ln_w, pair_ln_b, pair_eps, w_logits,
                                    w_vg, w_out, B, S, N, Cm, Cz, H, out, accumulate, workspace, s);
