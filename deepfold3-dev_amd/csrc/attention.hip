@@ -597,7 +597,8 @@ PF_DEVICE Frag16<float> buf_frag16<float>(__amdgpu_buffer_rsrc_t r, int voff, in
 // outputs finite -- and writes a per-wave flag redo[blockIdx.x * 4 + wave]; a flagged block
 // is recomputed by the exact mode (FAST = false with `redo` set), which runs the lazy
 // running-maximum softmax below and skips every block whose flags are all 0.
-template <class TC, int QS, bool O_HEAD_MAJOR, bool FAST, bool POST_SCALE = false, bool KMASK = true>
+template <class TC, int QS, bool O_HEAD_MAJOR, bool FAST, bool POST_SCALE = false, bool KMASK = true,
+          int HD = kHeadDim>
 __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2)) void tri_attn_kernel(
     const TC* __restrict__ Q, const TC* __restrict__ K, const TC* __restrict__ Vt, const float* __restrict__ PB,
     const float* __restrict__ MA, TC* __restrict__ O, int B, int N, int Np, int L, int Lp, int zero_masked_lines,
@@ -605,15 +606,18 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
     float* __restrict__ lse_out = nullptr) {
   constexpr int QB = 32 * QS;
   constexpr int NT = 64 * kLinesPerBlock;
-  constexpr int QLD = kHeadDim + (sizeof(TC) == 2 ? 0 : lds_pad<TC>());
+  constexpr int QLD = HD + (sizeof(TC) == 2 ? 0 : lds_pad<TC>());
   constexpr int QVEC = 16 / sizeof(TC);
-  auto qswz = [](int row) { return sizeof(TC) == 2 ? (row >> 2) & 3 : 0; };
+  static_assert(HD == 32 || (HD == 16 && sizeof(TC) == 2), "head dimension 32, or 16 in bf16");
+  // HD 16: Vt has 16 rows, and rows 16 .. 31 of its operand are ones, so P V^T also sums P
+  constexpr bool ONES = HD == 16;
+  auto qswz = [](int row) { return sizeof(TC) != 2 ? 0 : HD == 16 ? (row >> 3) & 1 : (row >> 2) & 3; };
   constexpr int TILE = QB * 32;                   // floats per bias stage: QB rows of 32 slots
   constexpr int DL = TILE * 4 / (NT * 16);        // direct loads per lane per stage
   static_assert(DL * NT * 16 == TILE * 4, "bias stage must split evenly over the block");
   constexpr int NSET = attn_kv_sets<TC>();
   // vmcnt budget: loads a lane issues per key block (bias stage + K + V [+ mask slot])
-  constexpr int KV_LOADS = (sizeof(TC) == 2 ? 4 : 8) + (KMASK ? 1 : 0);
+  constexpr int KV_LOADS = (ONES ? 3 : sizeof(TC) == 2 ? 4 : 8) + (KMASK ? 1 : 0);
   // The bias ring is dynamic LDS (attn_bias_lds_bytes at launch): the stage a step reads
   // is never the one its direct loads fill, and the explicit vmcnt + barrier order them.
   extern __shared__ __attribute__((aligned(16))) float bias_lds[];
@@ -646,9 +650,9 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
   const int lq = l & 31;
   const int hf = l >> 5;
   const size_t lineq = (size_t)b * Lp + (active ? line : lg * kLinesPerBlock);
-  const TC* Qh = Q + (lineq * kHeads + h) * (size_t)Np * kHeadDim;
-  const TC* Kh = K + (lineq * kHeads + h) * (size_t)Np * kHeadDim;
-  const TC* Vh = Vt + (lineq * kHeads + h) * (size_t)kHeadDim * Np;
+  const TC* Qh = Q + (lineq * kHeads + h) * (size_t)Np * HD;
+  const TC* Kh = K + (lineq * kHeads + h) * (size_t)Np * HD;
+  const TC* Vh = Vt + (lineq * kHeads + h) * (size_t)HD * Np;
   const float* PBh = PB + ((size_t)b * kHeads + h) * (size_t)Np * Np;
   const float* MAl = MA + lineq * Np;
   const int q0 = qb * QB;
@@ -659,15 +663,15 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
   // Np (K and V zero there), which add nothing.
   const int kb_last = KMASK ? nkb - 1 : Np / 32 - 1;
 
-  const auto rk = buf_rsrc(Kh, (unsigned)(Np * kHeadDim * sizeof(TC)));
-  const auto rv = buf_rsrc(Vh, (unsigned)(kHeadDim * Np * sizeof(TC)));
+  const auto rk = buf_rsrc(Kh, (unsigned)(Np * HD * sizeof(TC)));
+  const auto rv = buf_rsrc(Vh, (unsigned)(HD * Np * sizeof(TC)));
   const auto rm = buf_rsrc(MAl, (unsigned)(Np * sizeof(float)));
   const auto rb = buf_rsrc(PBh, (unsigned)((size_t)Np * Np * sizeof(float)));
   // bf16: K and Vt in 2 KB fragment-native key-block tiles; fp32: K [key][d], Vt [d][slot].
   constexpr bool kBlk = sizeof(TC) == 2;
-  const int k_voff = kBlk ? 16 * l : (lq * kHeadDim + 16 * hf) * (int)sizeof(TC);
-  const int v_voff = kBlk ? 16 * l : (lq * Np + 16 * hf) * (int)sizeof(TC);
-  const int v_kstride = kBlk ? kHeadDim * (int)sizeof(TC) : (int)sizeof(TC);  // bytes per key
+  const int k_voff = kBlk ? 16 * l : (lq * HD + 16 * hf) * (int)sizeof(TC);
+  const int v_voff = ONES ? 16 * (16 * hf + lq) : kBlk ? 16 * l : (lq * Np + 16 * hf) * (int)sizeof(TC);
+  const int v_kstride = kBlk ? HD * (int)sizeof(TC) : (int)sizeof(TC);  // bytes per key
   const int m_voff = key_slot(lq) * 4;
   // Bias stage: DL loads per lane, each 8 rows x 128 B; lane l writes row 8 blk + l / 8 at
   // physical chunk l % 8 = logical chunk (l % 8) ^ swz(row).
@@ -690,10 +694,25 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
 #pragma unroll
     for (int j = 0; j < DL; ++j) buf_load_lds16(rb, st + (w * DL + j) * 8 * 32, b_voff[j], soff);
   };
+  // HD 16: the lanes of Vt's rows load; the others keep the ones their registers start with
+  auto v16_load = [&](int k0, Frag16<TC>& vf) {
+    if constexpr (ONES) {
+      if (lq < 16) {
+        vf.v[0] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rv, v_voff, k0 * v_kstride, 0));
+        vf.v[1] =
+            __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rv, v_voff + 512, k0 * v_kstride, 0));
+      }
+    }
+  };
   auto kv_load = [&](int kb, Frag16<TC>& kf, Frag16<TC>& vf, float& mf) {
     const int k0 = min(kb, kb_last) * 32;
-    kf = buf_frag16<TC>(rk, k_voff, k0 * kHeadDim * (int)sizeof(TC));
-    vf = buf_frag16<TC>(rv, v_voff, k0 * v_kstride);
+    if constexpr (ONES) {
+      kf.v[0] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rk, k_voff, k0 * HD * 2, 0));
+      v16_load(k0, vf);
+    } else {
+      kf = buf_frag16<TC>(rk, k_voff, k0 * HD * (int)sizeof(TC));
+      vf = buf_frag16<TC>(rv, v_voff, k0 * v_kstride);
+    }
     if constexpr (KMASK)
       mf = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rm, m_voff, k0 * 4, 0));
     else
@@ -704,12 +723,12 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
   TC* qw = q_lds[w];
   if (active) {
 #pragma unroll
-    for (int it = 0; it < QB * kHeadDim / QVEC / 64; ++it) {
+    for (int it = 0; it < QB * HD / QVEC / 64; ++it) {
       const int idx = l + it * 64;
-      const int qq = idx / (kHeadDim / QVEC);
-      const int d0 = (idx % (kHeadDim / QVEC)) * QVEC;
+      const int qq = idx / (HD / QVEC);
+      const int d0 = (idx % (HD / QVEC)) * QVEC;
       *reinterpret_cast<u32x4*>(qw + qq * QLD + QVEC * ((d0 / QVEC) ^ qswz(qq))) =
-          *reinterpret_cast<const u32x4*>(Qh + (size_t)(q0 + qq) * kHeadDim + d0);
+          *reinterpret_cast<const u32x4*>(Qh + (size_t)(q0 + qq) * HD + d0);
     }
   }
   // Scan of the line's mask slots: 16-byte loads, four per lane in flight before any is
@@ -757,6 +776,12 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
   // insertion, which otherwise waits on the newest loads inside the first step of every round.
   Frag16<TC> kr[NSET], vr[NSET];
   float mr[NSET];
+  if constexpr (ONES) {
+#pragma unroll
+    for (int n = 0; n < NSET; ++n)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) vr[n].v[0][e] = vr[n].v[1][e] = (bf16)1.f;
+  }
   if (NSET == 3) kv_load(0, kr[0], vr[0], mr[0]);
   __builtin_amdgcn_sched_barrier(0);
   bias_issue(0, 0);
@@ -798,10 +823,15 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
         for (int e = 0; e < 4; ++e) sacc[4 * i + e] = bv[e];
       }
       if constexpr (KMASK) mma_mask(sacc, mk, TC{});
-      Frag16<TC> qf;
-      qf.v[0] = *reinterpret_cast<const bf16x8*>(qw + R * QLD + 8 * ((2 * hf) ^ qswz(R)));
-      qf.v[1] = *reinterpret_cast<const bf16x8*>(qw + R * QLD + 8 * ((2 * hf + 1) ^ qswz(R)));
-      mma32_16(sacc, kf, qf);
+      if constexpr (ONES) {
+        const bf16x8 qf = *reinterpret_cast<const bf16x8*>(qw + R * QLD + 8 * (hf ^ qswz(R)));
+        sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf.v[0], qf, sacc, 0, 0, 0);
+      } else {
+        Frag16<TC> qf;
+        qf.v[0] = *reinterpret_cast<const bf16x8*>(qw + R * QLD + 8 * ((2 * hf) ^ qswz(R)));
+        qf.v[1] = *reinterpret_cast<const bf16x8*>(qw + R * QLD + 8 * ((2 * hf + 1) ^ qswz(R)));
+        mma32_16(sacc, kf, qf);
+      }
     } else {
       // fp32: q k^T from a zero accumulator (sixteen 32x32x2 steps), then the bias, then
       // the key mask -- the eager order (q k^T scale + bias) + mask. Accumulating the
@@ -836,7 +866,9 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
 #pragma unroll
       for (int r = 0; r < 16; ++r) sacc[r] = __builtin_amdgcn_exp2f(sacc[r]);
       const Frag16<TC> pf = pack_p(sacc, TC{});
-      if constexpr (sizeof(TC) == 2) {
+      if constexpr (ONES) {
+        // row sums: rows 16 .. 31 of O^T below
+      } else if constexpr (sizeof(TC) == 2) {
         typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
         const bf16x2_t one2 = {(bf16)1.f, (bf16)1.f};
 #pragma unroll
@@ -948,7 +980,13 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
     // weighs 1 (the eager rule's uniform average); V is summed outside the bias ring.
     for (int kb = 0; kb < nkb; ++kb) {
       const int k0 = kb * 32;
-      const Frag16<TC> vf = buf_frag16<TC>(rv, v_voff, k0 * v_kstride);
+      Frag16<TC> vf;
+      if constexpr (ONES) {
+        vf = vr[0];  // the lanes past Vt's rows hold ones
+        v16_load(k0, vf);
+      } else {
+        vf = buf_frag16<TC>(rv, v_voff, k0 * v_kstride);
+      }
       f32x16 pr;
 #pragma unroll
       for (int r = 0; r < 16; ++r) pr[r] = k0 + 8 * (r >> 2) + 4 * hf + (r & 3) < N ? 1.f : 0.f;
@@ -967,6 +1005,13 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
   // fully masked line.
 #pragma unroll
   for (int s = 0; s < QS; ++s) lrun[s] += lsum[s][0] + lsum[s][1];
+  // row sum of query sub-block s
+  auto row_sum = [&](int s) -> float {
+    if constexpr (ONES)
+      return o[s][8];
+    else
+      return lrun[s] + __shfl_xor(lrun[s], 32, 64);
+  };
   // The last steps loaded repeat tiles into LDS; none may land after the block's LDS is
   // handed to another block.
   __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
@@ -975,7 +1020,7 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
     if (active) {
 #pragma unroll
       for (int s = 0; s < QS; ++s) {
-        const float lt = lrun[s] + __shfl_xor(lrun[s], 32, 64);
+        const float lt = row_sum(s);
         const bool real = q0 + 32 * s + lq < N;
         bad |= real && !(lt >= 0x1p-90f && lt <= 3.0e38f);
 #pragma unroll
@@ -992,7 +1037,7 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
   const bool write_zero = zero_masked_lines && all_masked;
 #pragma unroll
   for (int s = 0; s < QS; ++s) {
-    const float lt = lrun[s] + __shfl_xor(lrun[s], 32, 64);
+    const float lt = row_sum(s);
     const float inv = write_zero ? 0.f : 1.0f / lt;
     const int q = q0 + 32 * s + lq;
     if (q >= N) continue;
@@ -1006,11 +1051,11 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
     TC* dst;
     if constexpr (O_HEAD_MAJOR)
       dst = ost.n ? O + b * ost.b + line * ost.s + h * ost.h + q * ost.n
-                  : O + ((lineq * kHeads + h) * (size_t)N + q) * kHeadDim;
+                  : O + ((lineq * kHeads + h) * (size_t)N + q) * HD;
     else
-      dst = O + (lineq * (size_t)Np + q) * kC + h * kHeadDim;
+      dst = O + (lineq * (size_t)Np + q) * kC + h * HD;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < HD / 8; ++j) {
       float v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = o[s][4 * j + e] * inv;
@@ -1692,9 +1737,9 @@ int evo_attn_launch(const void* q, const void* k, const void* v, const float* re
 }
 
 // ------------------------------------------------------------------ generic channels / heads
-// GridSelfAttention for (C, H) other than (128, 4): the template stack's 64 channels in 4
-// heads of 16 and the 256-channel trunk's 8 heads of 32 (attention.py:56-269, head dim
-// max(C / H, 16), at most 32 here). Composed from the row kernels and the flash kernel:
+// GridSelfAttention for (C, H) other than (128, 4) (attention.py:56-269, head dim
+// max(C / H, 16), at most 32 here); in bf16, 64 channels in 4 heads and 256 in 8 have kernels
+// of their own below. Composed from the row kernels and the flash kernel:
 // LN(z) -> [q | k | v | g | pair bias] projection -> pack into groups of four heads, the head
 // dimension zero-padded to 32 (the logits and outputs are those of the real dimensions),
 // the line mask 1e9 (m - 1) and the pair bias [h][q][k] of the un-transposed positions ->
@@ -2272,11 +2317,332 @@ int grid_attn256_launch(const void* z, const float* mask, const float* lnw, cons
   return tile_gemm_rows_gated(og, G, wo, out, M, Cfg::C, HD, accumulate, sizeof(TZ) == 2 ? PF_BF16 : PF_F32, s);
 }
 
+// ------------------------------------------------------------------ 64 channels, 4 heads
+// GridSelfAttention at 64 channels in 4 heads of 16 with bf16 GEMMs (the template stack,
+// config.py:636-650). The weights of either projection fit one wave's registers, so both
+// kernels are streams of 16-position tiles, a tile per wave with no LDS tile and no barrier:
+// a lane holds 16 consecutive channels of one position (lanes l, l ^ 16, l ^ 32, l ^ 48
+// together its row), LayerNorms them and feeds them to 16x16x32 MFMAs as they are -- the
+// order of the contraction is free as long as the weight fragments follow it -- and every
+// accumulator layout is stored as it falls, in runs of 256 bytes and more:
+//   project64: q (scaled by d^-1/2 log2 e), k and Vt in the flash kernel's 16-wide frame (K
+//     and Vt in 1 KB key-block tiles: chunk 32 c + key holds dims 8 c .. of a key, chunk 32 j +
+//     16 hf + d slots 16 hf + 8 j .. of dim d), the pair bias and the line mask.
+//   out64: gate (recomputed from the z rows the residual needs), o * gate, output projection
+//     and residual; the product o * gate is the next MFMA's operand in its accumulator layout.
+// The flash kernel runs with head dimension 16: one q k^T MFMA instead of two, half the K
+// and V bytes, and the row sums from the ones that fill V's operand.
+// Both are bound by memory: 20 and 19 us at N=384 (78 and 57 MB), the flash kernel 50 us; the
+// composed path (LayerNorm, row GEMMs, five repacking passes, the flash kernel at dimension 32:
+// 72 us) took 271 us per direction.
+struct Grid64 {
+  static constexpr int C = 64, H = 4, D = 16;
+  static constexpr int NW = 4;  // waves per block
+};
+
+struct Grid64Ws {
+  size_t q, k, v, o, pb, ma, redo, total;
+};
+
+bool grid64_applies(int C, int H, int cdtype) { return C == Grid64::C && H == Grid64::H && cdtype == PF_BF16; }
+
+Grid64Ws grid64_layout(int B, int N) {
+  const size_t Np = pf::round_up((size_t)N, kPad);
+  const size_t tok = (size_t)B * N * Grid64::H * Np * Grid64::D * 2;
+  Grid64Ws w;
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = off;
+    off += pf::round_up(bytes, 256);
+    return at;
+  };
+  w.q = take(tok);
+  w.k = take(tok);
+  w.v = take(tok);
+  w.o = take(tok);
+  w.pb = take((size_t)B * Grid64::H * Np * Np * 4);
+  w.ma = take((size_t)B * N * Np * 4);
+  w.redo = take(redo_flag_bytes(B, N, (int)Np));
+  w.total = off;
+  return w;
+}
+
+// 16 consecutive channels of a row (raw) -> LayerNorm over the row's four lanes -> two B operands.
+template <class TZ>
+PF_DEVICE void ln64(const u32x4 (&raw)[sizeof(TZ)], const float* lnp, int c0, float eps, bf16x8 (&xf)[2]) {
+  constexpr int ZV = 16 / sizeof(TZ);
+  float v[16];
+#pragma unroll
+  for (int q = 0; q < (int)sizeof(TZ); ++q) unpack16<TZ>(raw[q], *reinterpret_cast<float(*)[ZV]>(v + ZV * q));
+  float s = 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) s += v[e];
+  s += __shfl_xor(s, 16, 64);
+  s += __shfl_xor(s, 32, 64);
+  const float mean = s * (1.0f / 64);
+  float qs = 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const float d = v[e] - mean;
+    qs += d * d;
+  }
+  qs += __shfl_xor(qs, 16, 64);
+  qs += __shfl_xor(qs, 32, 64);
+  const float rstd = rsqrtf(qs * (1.0f / 64) + eps);
+#pragma unroll
+  for (int e = 0; e < 16; ++e) xf[e >> 3][e & 7] = (bf16)((v[e] - mean) * rstd * lnp[c0 + e] + lnp[64 + c0 + e]);
+}
+
+template <class TZ>
+__global__ __launch_bounds__(64 * Grid64::NW, 2) void grid_project64_kernel(
+    const TZ* __restrict__ z, const float* __restrict__ mask, const float* __restrict__ lnw,
+    const float* __restrict__ lnb, float eps, const bf16* __restrict__ w5, bf16* __restrict__ Q,
+    bf16* __restrict__ K, bf16* __restrict__ Vt, float* __restrict__ PB, float* __restrict__ MA, int B, int N, int Np,
+    int transpose, float qscale) {
+  constexpr int C = Grid64::C, H = Grid64::H, D = Grid64::D;
+  constexpr int NLD = (int)sizeof(TZ);  // 16-byte loads of a lane's 16 channels
+  __shared__ __attribute__((aligned(16))) float lnp[2 * C];
+  const int l = lane_id();
+  const int r = l & 15, part = l >> 4;
+  if (threadIdx.x < C) {
+    lnp[threadIdx.x] = lnw[threadIdx.x];
+    lnp[C + threadIdx.x] = lnb[threadIdx.x];
+  }
+  bf16x8 wf[3 * H][2], wb[2];  // rows kind * 64 + 16 head + r, and the bias rows
+#pragma unroll
+  for (int t = 0; t < 3 * H; ++t)
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      wf[t][ks] = *reinterpret_cast<const bf16x8*>(w5 + (size_t)(16 * t + r) * C + 16 * part + 8 * ks);
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+    wb[ks] = *reinterpret_cast<const bf16x8*>(w5 + (size_t)(4 * C + r) * C + 16 * part + 8 * ks);
+  __syncthreads();
+
+  const int tpl = Np / 16;
+  const int ntiles = B * N * tpl;  // (2^31 tiles would be 4 TB of z)
+  const int step = (int)gridDim.x * Grid64::NW;
+  u32x4 zr[NLD];
+  float mk = 0.f;
+  auto issue = [&](int tile) __attribute__((always_inline)) {
+    const int bl = tile / tpl;
+    const int t = min((tile - bl * tpl) * 16 + r, N - 1);  // a token past N reads the last one
+    const int b = bl / N, line = bl - b * N;
+    const size_t pos = (size_t)b * N * N + (transpose ? (size_t)t * N + line : (size_t)line * N + t);
+#pragma unroll
+    for (int q = 0; q < NLD; ++q) zr[q] = *reinterpret_cast<const u32x4*>(z + pos * C + 16 * part + 16 / NLD * q);
+    if (part == 1) mk = mask[pos];
+  };
+  int tile = (int)blockIdx.x * Grid64::NW + wave_id();
+  if (tile < ntiles) issue(tile);
+  for (; tile < ntiles; tile += step) {
+    const int bl = tile / tpl;  // b N + line
+    const int t0 = (tile - bl * tpl) * 16;
+    const int t = t0 + r;
+    const int b = bl / N;
+    const int line = bl - b * N;
+    bf16x8 xf[2];
+    asm volatile("" ::: "memory");  // LayerNorm parameters from LDS per tile, not 32 registers
+    ln64<TZ>(zr, lnp, 16 * part, eps, xf);
+    const float mcur = mk;
+    if (tile + step < ntiles) issue(tile + step);
+    const float keep = t < N ? 1.f : 0.f;
+    const int blk = t0 & ~31, a = (t0 >> 4) & 1;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const size_t row = ((size_t)bl * H + h) * Np;
+      f32x4 q = {0.f, 0.f, 0.f, 0.f}, k = q, v = q;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        q = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][ks], xf[ks], q, 0, 0, 0);
+        k = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[H + h][ks], xf[ks], k, 0, 0, 0);
+        v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[ks], wf[2 * H + h][ks], v, 0, 0, 0);
+      }
+      // q, k: dims 4 part + e of token r; v: dim r of tokens 4 part + e (consecutive slots)
+      float qv[4], kv[4], vv[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        qv[e] = q[e] * qscale;
+        kv[e] = t < N ? k[e] : 0.f;
+        vv[e] = t0 + 4 * part + e < N ? v[e] : 0.f;
+      }
+      store_vec<bf16, 4>(Q + (row + t) * D + 4 * part, qv);
+      store_vec<bf16, 4>(K + (row + blk) * D + (32 * (part >> 1) + 16 * a + r) * 8 + 4 * (part & 1), kv);
+      store_vec<bf16, 4>(Vt + (row + blk) * D + (32 * a + 16 * (part & 1) + r) * 8 + 4 * (part >> 1), vv);
+    }
+    f32x4 p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[ks], xf[ks], p, 0, 0, 0);
+    const int slot = (t & ~31) + key_slot(t & 31);
+    if (part == 0) {  // the bias rows are heads 0..3
+#pragma unroll
+      for (int h = 0; h < H; ++h)
+        PB[(((size_t)b * H + h) * Np + line) * Np + (transpose ? t : slot)] = p[h] * kLog2e * keep;
+    } else if (part == 1) {
+      MA[(size_t)bl * Np + slot] = t < N ? (mcur - 1.0f) * 1e9f * kLog2e : -INFINITY;
+    }
+  }
+}
+
+template <class TZ>
+__global__ __launch_bounds__(64 * Grid64::NW, 3) void grid_out64_kernel(
+    const bf16* __restrict__ O, const bf16* __restrict__ Wg, const bf16* __restrict__ Wo, const TZ* z,
+    const float* __restrict__ lnw, const float* __restrict__ lnb, float eps, TZ* out, int B, int N, int Np,
+    int transpose, int accumulate, int res_is_z) {
+  constexpr int C = Grid64::C, H = Grid64::H, D = Grid64::D;
+  constexpr int NLD = (int)sizeof(TZ);
+  constexpr int ZV = 16 / NLD;
+  __shared__ __attribute__((aligned(16))) float lnp[2 * C];
+  const int l = lane_id();
+  const int r = l & 15, part = l >> 4;
+  if (threadIdx.x < C) {
+    lnp[threadIdx.x] = lnw[threadIdx.x];
+    lnp[C + threadIdx.x] = lnb[threadIdx.x];
+  }
+  // Gate rows 16 h + r over the lane's channel order. Output row r of tile t is channel 16 (r /
+  // 4) + 4 t + r % 4, so a lane's accumulators are 16 consecutive channels of its position; its
+  // columns follow o * gate: elements (head 2 ks, dim 4 part + e), then (head 2 ks + 1, ...).
+  bf16x8 wg[H][2], wo[4][2];
+#pragma unroll
+  for (int h = 0; h < H; ++h)
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      wg[h][ks] = *reinterpret_cast<const bf16x8*>(Wg + (size_t)(D * h + r) * C + 16 * part + 8 * ks);
+      const bf16* w = Wo + (size_t)(16 * (r >> 2) + 4 * h + (r & 3)) * C + 32 * ks + 4 * part;
+      const bf16x4 lo = *reinterpret_cast<const bf16x4*>(w), hi = *reinterpret_cast<const bf16x4*>(w + 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) wo[h][ks][e] = lo[e], wo[h][ks][4 + e] = hi[e];
+    }
+  __syncthreads();
+
+  const int tpl = (N + 15) / 16;
+  const int ntiles = B * N * tpl;  // (2^31 tiles would be 4 TB of z)
+  const int step = (int)gridDim.x * Grid64::NW;
+  u32x4 zr[NLD];
+  bf16x4 orr[H];
+  auto zpos = [&](int bl, int t) {
+    const int b = bl / N, line = bl - b * N;
+    return (size_t)b * N * N + (transpose ? (size_t)t * N + line : (size_t)line * N + t);
+  };
+  auto issue = [&](int tile) __attribute__((always_inline)) {
+    const int bl = tile / tpl;
+    const int t = min((tile - bl * tpl) * 16 + r, N - 1);
+    const size_t pos = zpos(bl, t);
+#pragma unroll
+    for (int q = 0; q < NLD; ++q) zr[q] = *reinterpret_cast<const u32x4*>(z + pos * C + 16 * part + ZV * q);
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+      orr[h] = *reinterpret_cast<const bf16x4*>(O + (((size_t)bl * H + h) * Np + t) * D + 4 * part);
+  };
+  int tile = (int)blockIdx.x * Grid64::NW + wave_id();
+  if (tile < ntiles) issue(tile);
+  for (; tile < ntiles; tile += step) {
+    const int bl = tile / tpl;
+    const int t = (tile - bl * tpl) * 16 + r;
+    bf16x8 xf[2], af[2];
+    asm volatile("" ::: "memory");  // as in project64
+    ln64<TZ>(zr, lnp, 16 * part, eps, xf);
+    float zv[16];
+#pragma unroll
+    for (int q = 0; q < NLD; ++q) unpack16<TZ>(zr[q], *reinterpret_cast<float(*)[ZV]>(zv + ZV * q));
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      f32x4 g = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wg[h][ks], xf[ks], g, 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) af[h >> 1][4 * (h & 1) + e] = (bf16)((float)orr[h][e] * sigmoidf_(g[e]));
+    }
+    if (tile + step < ntiles) issue(tile + step);
+    float y[16];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wo[m][ks], af[ks], acc, 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[4 * m + e] = acc[e];
+    }
+    if (t >= N) continue;
+    TZ* op = out + zpos(bl, t) * C + 16 * part;
+    if (accumulate) {
+      if (!res_is_z) {
+#pragma unroll
+        for (int q = 0; q < NLD; ++q) load16<TZ>(op + ZV * q, *reinterpret_cast<float(*)[ZV]>(zv + ZV * q));
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) y[e] += zv[e];
+    }
+#pragma unroll
+    for (int q = 0; q < NLD; ++q) store_vec<TZ, ZV>(op + ZV * q, y + ZV * q);
+  }
+}
+
+template <class TZ>
+int grid_attn64_launch(const void* z, const float* mask, const float* lnw, const float* lnb, float eps,
+                       const void* w5, const void* wo, int B, int N, int transpose, void* out, int accumulate,
+                       void* ws, hipStream_t s) {
+  constexpr int H = Grid64::H, D = Grid64::D, NW = Grid64::NW;
+  const int Np = (int)pf::round_up((size_t)N, kPad);
+  const Grid64Ws L = grid64_layout(B, N);
+  char* base = reinterpret_cast<char*>(ws);
+  bf16* Q = reinterpret_cast<bf16*>(base + L.q);
+  bf16* K = reinterpret_cast<bf16*>(base + L.k);
+  bf16* V = reinterpret_cast<bf16*>(base + L.v);
+  bf16* O = reinterpret_cast<bf16*>(base + L.o);
+  float* PB = reinterpret_cast<float*>(base + L.pb);
+  float* MA = reinterpret_cast<float*>(base + L.ma);
+  int* redo = reinterpret_cast<int*>(base + L.redo);
+  {
+    const long nblk = ((long)B * N * (Np / 16) + NW - 1) / NW;
+    grid_project64_kernel<TZ><<<(unsigned)std::min<long>(nblk, 2L * pf::cu_count()), 64 * NW, 0, s>>>(
+        (const TZ*)z, mask, lnw, lnb, eps, (const bf16*)w5, Q, K, V, PB, MA, B, N, Np, transpose,
+        (1.0f / sqrtf((float)D)) * kLog2e);
+    if (int e = pf::check_launch("grid_project64")) return e;
+  }
+  if (Np > N) {
+    const long n4 = (long)(Np - N) * Np / 4;
+    pb_zero_pad_rows_kernel<<<dim3((unsigned)std::min<long>((n4 + 255) / 256, 64), B * H), 256, 0, s>>>(PB, N, Np);
+    if (int e = pf::check_launch("pb_zero_pad_rows")) return e;
+  }
+  if (transpose) {
+    const int nt = Np / 32;
+    pb_transpose_kernel<<<dim3(nt * (nt + 1) / 2, B * H), 256, 0, s>>>(PB, Np, nullptr, N);
+    if (int e = pf::check_launch("pb_transpose")) return e;
+  }
+  constexpr int QS = attn_qsub<bf16>();
+  constexpr int NT = 64 * kLinesPerBlock;
+  const int nqb = Np / (32 * QS);
+  const int nlg = (N + kLinesPerBlock - 1) / kLinesPerBlock;
+  const long total = (long)B * nlg * H * nqb;
+  const int remap = (total % 8 == 0) ? 1 : 0;
+  const Strides4 so{(long)N * H * Np * D, (long)H * Np * D, (long)Np * D, (long)D};
+  const dim3 grid((unsigned)total);
+  constexpr size_t lds = attn_bias_lds_bytes<bf16>();
+  pf::KernelTimer timer("tri_attn", s);
+  tri_attn_kernel<bf16, QS, true, true, false, true, D><<<grid, NT, lds, s>>>(Q, K, V, PB, MA, O, B, N, Np, N, N, 0,
+                                                                              remap, redo, 1.f, so);
+  timer.stop();
+  if (int e = pf::check_launch("tri_attn")) return e;
+  tri_attn_kernel<bf16, QS, true, false, false, true, D><<<grid, NT, lds, s>>>(Q, K, V, PB, MA, O, B, N, Np, N, N, 0,
+                                                                               remap, redo, 1.f, so);
+  if (int e = pf::check_launch("tri_attn_redo")) return e;
+  const long nblk = ((long)B * N * ((N + 15) / 16) + NW - 1) / NW;
+  const bf16* wg = (const bf16*)w5 + (size_t)3 * Grid64::C * Grid64::C;
+  grid_out64_kernel<TZ><<<(unsigned)std::min<long>(nblk, 3L * pf::cu_count()), 64 * NW, 0, s>>>(
+      O, wg, (const bf16*)wo, (const TZ*)z, lnw, lnb, eps, (TZ*)out, B, N, Np, transpose, accumulate,
+      out == z ? 1 : 0);
+  return pf::check_launch("grid_out64");
+}
+
 template <class TZ, class TC>
 int grid_attn_generic_launch(const void* z, const float* mask, const float* lnw, const float* lnb, float eps,
                              const void* w5, const void* wo, int B, int N, int C, int H, int transpose, void* out,
                              int accumulate, const float* key_mask, void* ws, hipStream_t s) {
   const int cd = sizeof(TC) == 4 ? PF_F32 : PF_BF16;
+  if constexpr (sizeof(TC) == 2)
+    if (grid64_applies(C, H, cd))
+      return grid_attn64_launch<TZ>(z, mask, lnw, lnb, eps, w5, wo, B, N, transpose, out, accumulate, ws, s);
   if constexpr (sizeof(TC) == 2)
     if (grid256_applies(C, H, cd))
       return grid_attn256_launch<TZ>(z, mask, lnw, lnb, eps, w5, wo, B, N, transpose, out, accumulate, key_mask, ws,
@@ -2359,6 +2725,7 @@ extern "C" {
 size_t pf_grid_attn_workspace_bytes(int B, int N, int C, int H, int cdtype) {
   if (B <= 0 || N <= 0) return 0;
   if (C == kC && H == kHeads) return attn_ws_layout(B, N, cdtype).total;
+  if (grid64_applies(C, H, cdtype)) return grid64_layout(B, N).total;
   if (grid256_applies(C, H, cdtype)) return grid256_layout(B, N).total;
   return grid_gen_supported(C, H) ? grid_gen_layout(B, N, C, H, cdtype).total : 0;
 }
@@ -2433,6 +2800,10 @@ int pf_grid_attn_redo_flags(int B, int N, int C, int H, int cdtype, size_t* offs
              PF_ERR_UNSUPPORTED, "pf_grid_attn_redo_flags: B=%d N=%d C=%d H=%d cdtype=%d", B, N, C, H, cdtype);
   // generic channels: the flags of the last group of four heads (256 channels: both groups)
   *count = redo_flag_count(B, N, pf::pad128(N), cdtype);
+  if (!fused && grid64_applies(C, H, cdtype)) {
+    *offset = grid64_layout(B, N).redo;
+    return pf::ok();
+  }
   if (!fused && grid256_applies(C, H, cdtype)) {
     const Grid256Ws L = grid256_layout(B, N);
     *offset = L.redo + L.gredo * sizeof(int);

@@ -1,0 +1,73 @@
+"""GPU: grid attention at 64 channels in 4 heads of 16 with bf16 GEMMs (the template stack;
+reference ``attention.py:56-269``, ``config.py:636-650``): the register-resident projection
+and output kernels and the flash kernel at head dimension 16. Rows and columns, token counts
+around the 16-position tiles and the 32-key blocks, per-line masks with fully masked lines,
+both streams, a batch of two, the in-place residual, and logits that overflow the fast softmax
+pass. Against the oracle in fp64 by the bf16 rule; batch items bit for bit independent."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import pairformer_ref as R
+from tests._helpers import assert_bf16_rule, mod, sub, to
+
+pytestmark = pytest.mark.gpu
+W = mod("weights")
+attention = mod("attention")
+_lib = mod("_lib")
+BF = torch.bfloat16
+C = 64
+
+
+def _module(dev, transpose, seed, bias_gain=1.0):
+    p = sub(W.make_block_weights(seed, perturb_affine=True, c_pair=C), "pair_attn_col." if transpose else "pair_attn_row.")
+    p["pair_bias.weight"] = p["pair_bias.weight"] * bias_gain
+    m = attention.GridSelfAttention(C, num_heads=4, transpose=transpose).eval()
+    m.load_state_dict(p)
+    return m.to(dev), p
+
+
+@pytest.mark.parametrize("transpose", [False, True], ids=["rows", "cols"])
+@pytest.mark.parametrize("stream", [BF, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("n,batch", [(1, 1), (15, 1), (16, 2), (17, 1), (33, 1), (128, 1), (150, 1)])
+def test_grid64(dev, n, batch, stream, transpose):
+    print(f"[grid64] N={n} batch={batch} {stream} transpose={transpose}", flush=True)
+    m, p = _module(dev, transpose, 40 + n)
+    g = torch.Generator().manual_seed(n)
+    z = torch.randn(batch, n, n, C, generator=g).to(dev, stream)
+    mask = (torch.rand(batch, n, n, generator=g) > 0.2).float()
+    if n > 2:
+        mask[:, 1] = 0.0  # a fully masked line in either direction
+        mask[:, :, 2] = 0.0
+    mask = mask.to(dev)
+    with torch.no_grad(), torch.autocast("cuda", dtype=BF, enabled=stream == torch.float32):
+        got = m(z, mask)
+        last = m(z[-1:], mask[-1:])
+        res = m.forward_residual_(z.clone(), mask)
+        eager = R.grid_attention(z.to(BF), mask, to(p, dev, BF), transpose)
+    ref = R.grid_attention(z.double(), mask.double(), to(p, dev, torch.float64), transpose)
+    assert got.dtype == stream and torch.equal(last, got[-1:])
+    print("   ", assert_bf16_rule(got.cpu(), eager.float().cpu(), ref.cpu(), f"grid64 N={n}"), flush=True)
+    want = z.double() + got.double()  # one rounding of z + update, against the separately rounded update
+    tol = (2.0**-7 if stream == BF else 2.0**-22) * want.abs().max().item()
+    assert (res.double() - want).abs().max().item() <= tol
+
+
+@pytest.mark.parametrize("transpose", [False, True], ids=["rows", "cols"])
+def test_grid64_exact_redo(dev, transpose):
+    """A pair bias of several hundred overflows 2^s: the exact pass must take those lines over."""
+    print(f"[grid64] exact redo transpose={transpose}", flush=True)
+    n = 70
+    m, p = _module(dev, transpose, 3, bias_gain=300.0)
+    z = torch.randn(1, n, n, C, generator=torch.Generator().manual_seed(4)).to(dev)
+    mask = torch.ones(1, n, n, device=dev)
+    mask[:, :, -5:] = 0.0 if not transpose else 1.0
+    with torch.no_grad(), torch.autocast("cuda", dtype=BF), _lib.RedoRecorder() as log:
+        got = m(z, mask)
+        eager = R.grid_attention(z.to(BF), mask, to(p, dev, BF), transpose)
+    ref = R.grid_attention(z.double(), mask.double(), to(p, dev, torch.float64), transpose)
+    assert sum(log) > 0, "the exact pass never ran"
+    assert bool(torch.isfinite(got).all())
+    assert_bf16_rule(got.cpu(), eager.float().cpu(), ref.cpu(), "grid64 redo")
