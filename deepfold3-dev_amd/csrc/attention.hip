@@ -2367,32 +2367,6 @@ Grid64Ws grid64_layout(int B, int N) {
   return w;
 }
 
-// 16 consecutive channels of a row (raw) -> LayerNorm over the row's four lanes -> two B operands.
-template <class TZ>
-PF_DEVICE void ln64(const u32x4 (&raw)[sizeof(TZ)], const float* lnp, int c0, float eps, bf16x8 (&xf)[2]) {
-  constexpr int ZV = 16 / sizeof(TZ);
-  float v[16];
-#pragma unroll
-  for (int q = 0; q < (int)sizeof(TZ); ++q) unpack16<TZ>(raw[q], *reinterpret_cast<float(*)[ZV]>(v + ZV * q));
-  float s = 0.f;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) s += v[e];
-  s += __shfl_xor(s, 16, 64);
-  s += __shfl_xor(s, 32, 64);
-  const float mean = s * (1.0f / 64);
-  float qs = 0.f;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const float d = v[e] - mean;
-    qs += d * d;
-  }
-  qs += __shfl_xor(qs, 16, 64);
-  qs += __shfl_xor(qs, 32, 64);
-  const float rstd = rsqrtf(qs * (1.0f / 64) + eps);
-#pragma unroll
-  for (int e = 0; e < 16; ++e) xf[e >> 3][e & 7] = (bf16)((v[e] - mean) * rstd * lnp[c0 + e] + lnp[64 + c0 + e]);
-}
-
 template <class TZ>
 __global__ __launch_bounds__(64 * Grid64::NW, 2) void grid_project64_kernel(
     const TZ* __restrict__ z, const float* __restrict__ mask, const float* __restrict__ lnw,

@@ -605,3 +605,32 @@ struct LnTile {
     }
   }
 };
+
+// LayerNorm of 64-channel rows in 16x16x32 operand registers: lane l holds channels c0 = 16 (l >> 4)
+// .. +15 of row l & 15 as loaded; the row's four lanes reduce together, and the 16 normalised
+// values are two operands (k order: the lane's own channels, which the other operand follows).
+// lnp: weight [64], then bias [64].
+template <class TZ>
+PF_DEVICE void ln64(const u32x4 (&raw)[sizeof(TZ)], const float* lnp, int c0, float eps, bf16x8 (&xf)[2]) {
+  constexpr int ZV = 16 / sizeof(TZ);
+  float v[16];
+#pragma unroll
+  for (int q = 0; q < (int)sizeof(TZ); ++q) unpack16<TZ>(raw[q], *reinterpret_cast<float(*)[ZV]>(v + ZV * q));
+  float s = 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) s += v[e];
+  s += __shfl_xor(s, 16, 64);
+  s += __shfl_xor(s, 32, 64);
+  const float mean = s * (1.0f / 64);
+  float qs = 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const float d = v[e] - mean;
+    qs += d * d;
+  }
+  qs += __shfl_xor(qs, 16, 64);
+  qs += __shfl_xor(qs, 32, 64);
+  const float rstd = rsqrtf(qs * (1.0f / 64) + eps);
+#pragma unroll
+  for (int e = 0; e < 16; ++e) xf[e >> 3][e & 7] = (bf16)((v[e] - mean) * rstd * lnp[c0 + e] + lnp[64 + c0 + e]);
+}
