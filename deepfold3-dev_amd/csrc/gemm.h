@@ -21,5 +21,5 @@ int tile_gemm_rows(const void* A, const void* W, void* out, long M, int Nout, in
 // gate [M][K] like A, each product rounded to bf16 before the GEMM.
 int tile_gemm_rows_gated(const void* A, const void* gate, const void* W, void* out, long M, int Nout, int K,
                          int accumulate, int out_dtype, hipStream_t s);
-// Rows from which the row GEMM hands over to tile_gemm_rows.
+// Rows from which the row GEMM always hands over to tile_gemm_rows.
 constexpr long kTileGemmMinRows = 16384;

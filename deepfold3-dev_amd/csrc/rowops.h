@@ -4,6 +4,9 @@
 // linkage), so each keeps its own instantiations.
 #pragma once
 
+#include <algorithm>
+#include <type_traits>
+
 #include "capi.h"
 #include "common.h"
 #include "gemm.h"
@@ -83,16 +86,17 @@ __global__ __launch_bounds__(256) void ln_rows_vec_kernel(const TI* __restrict__
 enum { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2 };
 
 // out = epi(A W^T [+ bias]); A [M][K], W [Nw][K] (TC, k contiguous). One block computes a
-// (16 RB)-row x 64-column output tile, each wave one 16-column block over RB row blocks;
-// the operands come straight from global memory (L2), four k-steps' loads in flight.
-// RB = 2 when the 64-row grid would leave most CUs idle (the single track has N rows).
+// 64-row x 64-column output tile, each wave one 16-column block over four row blocks; the
+// operands come straight from global memory (L2), four k-steps' loads in flight. What is left to
+// it: more rows than the small kernel's with a bias, or unaligned operands.
 // EPI_SWIGLU: output column j is silu(h_j) * h_{F + j} with F = Nout (W has 2 Nout rows).
 // bias (fp32, may be null) applies to the first nbias output columns (EPI_STORE only).
-template <class TC, class TO, int EPI, int RB>
+template <class TC, class TO, int EPI>
 __global__ __launch_bounds__(256) void rowgemm_kernel(const TC* __restrict__ A, const TC* __restrict__ W,
                                                       const float* __restrict__ bias, int nbias, TO* __restrict__ out,
                                                       long M, int Nout, int K) {
   using MF = Mfma<TC>;
+  constexpr int RB = 4;
   const int w = wave_id();
   const int l = lane_id();
   const long m0 = (long)blockIdx.x * 16 * RB;
@@ -151,6 +155,166 @@ __global__ __launch_bounds__(256) void rowgemm_kernel(const TC* __restrict__ A, 
     }
 }
 
+// The row GEMM for few rows (the single track: N tokens). Its time is one block's chain of
+// operand loads, so a block takes a 32 x 32 output tile and its four waves split K (steps w, w
+// + 4, ...), summed in wave order through LDS, which also turns the stores into row pieces;
+// with LN the A rows are LayerNormed into LDS first (re-done by every column block: 32 rows of
+// a few KB) instead of by a launch of their own. A 384-channel transition of 64 rows 31 -> 15 us
+// in bf16 and 73 -> 25 in fp32, of 384 rows 38 -> 20 and 89 -> 40 (LayerNorm launch and 32 x 64
+// tiles over the whole K per wave before).
+template <class TA, class TC, class TO, int EPI, bool LN>
+__global__ __launch_bounds__(256) void rowgemm_small_kernel(const TA* __restrict__ A, const float* __restrict__ lnw,
+                                                            const float* __restrict__ lnb, float eps,
+                                                            const TC* __restrict__ W, const float* __restrict__ bias,
+                                                            int nbias, TO* __restrict__ out, long M, int Nout, int K,
+                                                            int vec_out) {
+  using MF = Mfma<TC>;
+  constexpr int NA = EPI == EPI_SWIGLU ? 2 : 1;
+  constexpr int SLD = 36;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x;
+  const int w = wave_id();
+  const int l = lane_id();
+  const int r = l & 15, kq = (l >> 4) * MF::KPL;
+  const long m0 = (long)blockIdx.x * 32;
+  const int n0 = blockIdx.y * 32;
+  const int lda = LN ? K + lds_pad<TC>() : K;
+  TC* xs = reinterpret_cast<TC*>(smem);
+  if constexpr (LN) {  // 8 threads per row, 16-byte pieces
+    constexpr int VEC = 16 / sizeof(TA);
+    const int row = tid >> 3, sub = (tid & 7) * VEC;
+    const TA* src = A + min(m0 + row, M - 1) * K;
+    float v[VEC];
+    float s = 0.f;
+    for (int c = sub; c < K; c += 8 * VEC) {
+      load16<TA>(src + c, v);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) s += v[e];
+    }
+    const float mean = dpp_sum8(s) / K;
+    float q = 0.f;
+    for (int c = sub; c < K; c += 8 * VEC) {
+      load16<TA>(src + c, v);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        const float d = v[e] - mean;
+        q += d * d;
+      }
+    }
+    const float rstd = rsqrtf(dpp_sum8(q) / K + eps);
+    for (int c = sub; c < K; c += 8 * VEC) {
+      load16<TA>(src + c, v);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[e] = (v[e] - mean) * rstd * lnw[c + e] + lnb[c + e];
+      store_vec<TC, VEC>(xs + row * lda + c, v);
+    }
+    __syncthreads();
+  }
+  const TC* arow[2];
+  const TC* wrow[NA][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    arow[i] = LN ? xs + (16 * i + r) * lda + kq : reinterpret_cast<const TC*>(A) + min(m0 + 16 * i + r, M - 1) * K + kq;
+    // a tile's second column block may lie past Nout: it repeats the last rows, unused
+#pragma unroll
+    for (int a = 0; a < NA; ++a) wrow[a][i] = W + (size_t)(a * Nout + min(n0 + 16 * i + r, Nout - 1)) * K + kq;
+  }
+  f32x4 acc[NA][2][2];
+#pragma unroll
+  for (int a = 0; a < NA; ++a) zero_acc(acc[a]);
+  // groups of three steps with all their loads in flight (the track's K = 384 in bf16 is one
+  // group per wave), then single steps
+  auto steps = [&](int k0, auto count) __attribute__((always_inline)) {
+    constexpr int G = decltype(count)::value;
+    typename MF::Frag af[G][2], bf[G][NA][2];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int k = k0 + g * 4 * MF::K16;
+#pragma unroll
+      for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) bf[g][a][j] = MF::load(wrow[a][j] + k);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) af[g][i] = MF::load(arow[i] + k);
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) MF::mma16(acc[a][i][j], af[g][i], bf[g][a][j]);
+  };
+  int k0 = w * MF::K16;
+  for (; k0 + 8 * MF::K16 < K; k0 += 12 * MF::K16) steps(k0, std::integral_constant<int, 3>{});
+  for (; k0 < K; k0 += 4 * MF::K16) steps(k0, std::integral_constant<int, 1>{});
+  if constexpr (LN) __syncthreads();  // xs becomes the sums [wave][a][row][col]
+  float* st = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int a = 0; a < NA; ++a)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          st[((w * NA + a) * 32 + 16 * i + 4 * (l >> 4) + e) * SLD + 16 * j + r] = acc[a][i][j][e];
+  __syncthreads();
+  const int row = tid >> 3, c0 = (tid & 7) * 4;
+  const long m = m0 + row;
+  const int n = n0 + c0;
+  if (m >= M || n >= Nout) return;
+  f32x4 y[NA];
+#pragma unroll
+  for (int a = 0; a < NA; ++a) {
+    y[a] = *reinterpret_cast<const f32x4*>(st + (a * 32 + row) * SLD + c0);
+#pragma unroll
+    for (int v = 1; v < 4; ++v) y[a] += *reinterpret_cast<const f32x4*>(st + ((v * NA + a) * 32 + row) * SLD + c0);
+  }
+  TO* dst = out + m * Nout + n;
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = EPI == EPI_SWIGLU ? siluf_(y[0][e]) * y[NA - 1][e] : y[0][e];
+    if (EPI == EPI_RESIDUAL) v[e] += to_f32(dst[e]);
+    if (EPI == EPI_STORE && bias && n + e < nbias) v[e] += bias[n + e];
+  }
+  if (vec_out) {
+    store_vec<TO, 4>(dst, v);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dst[e] = from_f32<TO>(v[e]);
+  }
+}
+
+// Where the small kernel hands over to the tiled one: the tiled GEMM's time is a fixed chain per
+// k-tile until its grid fills the chip, the small one's grows with the M x Nw outputs computed
+// (Nw weight rows), so the line is a number of outputs. Transition of 384 channels: bf16 1536
+// rows (4.7 M outputs in W1) 49 against 49 us, 2048 rows 56 against 46; of 128 channels, factor 2:
+// 6144 rows (3.1 M) 14.7 against 16.1, 8192 18.1 against 16.6; fp32 384 channels 3072 rows (9.4 M)
+// 170 against 206, 4096 216 against 208; 128 channels 12288 rows (6.3 M) 48 against 53.
+template <class TC>
+bool rowgemm_small(long M, long Nw) {
+  return M < kTileGemmMinRows && M * Nw <= (sizeof(TC) == 2 ? 3500000L : 8000000L);
+}
+
+template <class TA, class TC, class TO, int EPI, bool LN>
+int rowgemm_small_launch(const void* A, const float* lnw, const float* lnb, float eps, const void* W,
+                         const float* bias, int nbias, void* out, long M, int Nout, int K, hipStream_t s) {
+  const int sums = 4 * (EPI == EPI_SWIGLU ? 2 : 1) * 32 * 36 * 4;
+  const int tile = LN ? 32 * (K + lds_pad<TC>()) * (int)sizeof(TC) : 0;
+  const int lds = std::max(sums, tile);
+  const void* fn = (const void*)rowgemm_small_kernel<TA, TC, TO, EPI, LN>;
+  const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  PF_REQUIRE(e == hipSuccess, PF_ERR_LAUNCH, "row gemm: cannot reserve %d bytes of LDS: %s", lds,
+             hipGetErrorString(e));
+  const int vec_out = pf::aligned16(out);  // Nout is a multiple of 16
+  rowgemm_small_kernel<TA, TC, TO, EPI, LN>
+      <<<dim3((unsigned)((M + 31) / 32), (unsigned)((Nout + 31) / 32)), 256, lds, s>>>(
+          (const TA*)A, lnw, lnb, eps, (const TC*)W, bias, nbias, (TO*)out, M, Nout, K, vec_out);
+  return pf::check_launch("rowgemm");
+}
 
 template <class TI, class TO>
 int ln_launch(const void* x, const float* w, const float* b, float eps, void* out, long M, int C, hipStream_t s) {
@@ -172,22 +336,27 @@ int ln_launch(const void* x, const float* w, const float* b, float eps, void* ou
 template <class TC, class TO, int EPI>
 int rowgemm_launch(const void* A, const void* W, const float* bias, int nbias, void* out, long M, int Nout, int K,
                    hipStream_t s) {
-  // Many rows (the pair paths at generic widths): the LDS-tiled GEMM with the same epilogue.
+  if (rowgemm_small<TC>(M, (EPI == EPI_SWIGLU ? 2L : 1L) * Nout))
+    return rowgemm_small_launch<TC, TC, TO, EPI, false>(A, nullptr, nullptr, 0.f, W, bias, nbias, out, M, Nout, K, s);
+  // More rows: the LDS-tiled GEMM with the same epilogues (it takes no bias).
   constexpr int kt = sizeof(TC) == 2 ? 32 : 16;  // tile_gemm_rows' k-tile
-  if (M >= kTileGemmMinRows && K % kt == 0 && (bias == nullptr || nbias == 0) && pf::aligned16(A) &&
-      pf::aligned16(W))
+  if (K % kt == 0 && (bias == nullptr || nbias == 0) && pf::aligned16(A) && pf::aligned16(W))
     return tile_gemm_rows(A, W, out, M, Nout, K, EPI, sizeof(TC) == 2 ? PF_BF16 : PF_F32,
                           sizeof(TO) == 2 ? PF_BF16 : PF_F32, s);
-  const long nb64 = ((M + 63) / 64) * ((Nout + 63) / 64);
-  if (nb64 < 2L * pf::cu_count()) {  // few row blocks: 32-row tiles, twice the blocks
-    dim3 grid((unsigned)((M + 31) / 32), (unsigned)((Nout + 63) / 64));
-    rowgemm_kernel<TC, TO, EPI, 2><<<grid, 256, 0, s>>>((const TC*)A, (const TC*)W, bias, nbias, (TO*)out, M, Nout, K);
-  } else {
-    dim3 grid((unsigned)((M + 63) / 64), (unsigned)((Nout + 63) / 64));
-    rowgemm_kernel<TC, TO, EPI, 4><<<grid, 256, 0, s>>>((const TC*)A, (const TC*)W, bias, nbias, (TO*)out, M, Nout, K);
-  }
+  dim3 grid((unsigned)((M + 63) / 64), (unsigned)((Nout + 63) / 64));
+  rowgemm_kernel<TC, TO, EPI><<<grid, 256, 0, s>>>((const TC*)A, (const TC*)W, bias, nbias, (TO*)out, M, Nout, K);
   return pf::check_launch("rowgemm");
 }
 
+// out = epi(LN(x) W^T [+ bias]) through the scratch rows xn [M][K]; few rows are LayerNormed
+// inside the GEMM. `out` must not overlap x (blocks read x rows while others store).
+template <class TI, class TC, class TO, int EPI>
+int ln_rowgemm_launch(const void* x, const float* lnw, const float* lnb, float eps, void* xn, const void* W,
+                      const float* bias, int nbias, void* out, long M, int Nout, int K, hipStream_t s) {
+  if (rowgemm_small<TC>(M, (EPI == EPI_SWIGLU ? 2L : 1L) * Nout) && pf::aligned16(x) && K <= 1024)
+    return rowgemm_small_launch<TI, TC, TO, EPI, true>(x, lnw, lnb, eps, W, bias, nbias, out, M, Nout, K, s);
+  if (int e = ln_launch<TI, TC>(x, lnw, lnb, eps, xn, M, K, s)) return e;
+  return rowgemm_launch<TC, TO, EPI>(xn, W, bias, nbias, out, M, Nout, K, s);
+}
 
 }  // namespace

@@ -257,8 +257,9 @@ int single_attn_launch(const void* s_in, const float* seq_mask, const float* pai
   TC* qkvg = reinterpret_cast<TC*>(p);
   p += pf::round_up((size_t)M * 4 * HD * sizeof(TC), 256);
   TC* og = reinterpret_cast<TC*>(p);
-  if (int e = ln_launch<TZ, TC>(s_in, lnw, lnb, eps, xn, M, C, st)) return e;
-  if (int e = rowgemm_launch<TC, TC, EPI_STORE>(xn, wqkvg, qbias, HD, qkvg, M, 4 * HD, C, st)) return e;
+  if (int e = ln_rowgemm_launch<TZ, TC, TC, EPI_STORE>(s_in, lnw, lnb, eps, xn, wqkvg, qbias, HD, qkvg, M, 4 * HD, C,
+                                                       st))
+    return e;
   {
     const int Np = (int)pf::round_up((size_t)N, 32);
     p += pf::round_up((size_t)M * HD * sizeof(TC), 256);
@@ -284,8 +285,7 @@ int single_attn_launch(const void* s_in, const float* seq_mask, const float* pai
 template <class TZ, class TC>
 int recycle_embed_launch(const void* prev, const float* lnw, const float* lnb, float eps, const void* w, long M,
                          int C, void* out, void* ws, hipStream_t st) {
-  if (int e = ln_launch<TZ, TC>(prev, lnw, lnb, eps, ws, M, C, st)) return e;
-  return rowgemm_launch<TC, TZ, EPI_RESIDUAL>(ws, w, nullptr, 0, out, M, C, C, st);
+  return ln_rowgemm_launch<TZ, TC, TZ, EPI_RESIDUAL>(prev, lnw, lnb, eps, ws, w, nullptr, 0, out, M, C, C, st);
 }
 
 template <class TZ, class TC>
@@ -296,8 +296,8 @@ int transition_generic_launch(const void* x, const float* lnw, const float* lnb,
   TC* xn = reinterpret_cast<TC*>(p);
   p += pf::round_up((size_t)M * C * sizeof(TC), 256);
   TC* u = reinterpret_cast<TC*>(p);
-  if (int e = ln_launch<TZ, TC>(x, lnw, lnb, eps, xn, M, C, st)) return e;
-  if (int e = rowgemm_launch<TC, TC, EPI_SWIGLU>(xn, w1, nullptr, 0, u, M, F, C, st)) return e;
+  if (int e = ln_rowgemm_launch<TZ, TC, TC, EPI_SWIGLU>(x, lnw, lnb, eps, xn, w1, nullptr, 0, u, M, F, C, st))
+    return e;
   if (accumulate) return rowgemm_launch<TC, TZ, EPI_RESIDUAL>(u, w2, nullptr, 0, out, M, C, F, st);
   return rowgemm_launch<TC, TZ, EPI_STORE>(u, w2, nullptr, 0, out, M, C, F, st);
 }

@@ -1,0 +1,78 @@
+"""GPU: the few-row GEMM behind the single track (``csrc/rowops.h``), through the transition
+(``primitives.py:193-251``) and LN + linear (``layernorm_linear.py:537-592``): row counts around
+its 32 x 32 tiles, output widths that leave half a tile, K steps that do not divide over the
+four waves, the hand-over to the tiled GEMM (3.5 M outputs in bf16, 8 M in fp32), a bias past it,
+and an unaligned input (LayerNorm launched on its own). fp32 against float64 at 1e-5; bf16 by
+the bf16 rule."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import pairformer_ref as R
+from tests._helpers import assert_bf16_rule, assert_fp32_close, mod, to
+
+pytestmark = pytest.mark.gpu
+primitives = mod("primitives")
+fused = mod("fused")
+BF = torch.bfloat16
+
+
+def _transition(dev, C, factor, seed):
+    g = torch.Generator().manual_seed(seed)
+    rn = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    p = {"norm.weight": 1 + 0.1 * rn(C), "norm.bias": 0.1 * rn(C), "linear1.weight": rn(2 * factor * C, C) / C**0.5,
+         "linear2.weight": rn(C, factor * C) / (factor * C) ** 0.5}  # fmt: skip
+    m = primitives.TransitionBlock(C, factor).eval()
+    m.load_state_dict(p)
+    return m.to(dev), p
+
+
+def _check(got, x, p, dev, what):
+    ref = R.transition(x.double(), to(p, dev, torch.float64))
+    if got.dtype == torch.float32:
+        assert_fp32_close(got.cpu(), ref.cpu(), what=what)
+    else:
+        eager = R.transition(x, to(p, dev, BF))
+        print("   ", assert_bf16_rule(got.float().cpu(), eager.float().cpu(), ref.cpu(), what), flush=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, BF], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("M,C,factor", [(1, 384, 4), (31, 384, 4), (33, 384, 4), (100, 96, 2), (64, 32, 2),
+                                        (1139, 384, 4), (1140, 384, 4), (2604, 384, 4), (2605, 384, 4)])  # fmt: skip
+def test_transition_few_rows(dev, M, C, factor, dtype):
+    print(f"[few rows] M={M} C={C} factor={factor} {dtype}", flush=True)
+    m, p = _transition(dev, C, factor, M + C)
+    x = torch.randn(M, C, generator=torch.Generator().manual_seed(M)).to(dev, dtype)
+    with torch.no_grad():
+        got = m.to(dtype)(x)
+        res, _ = m.forward_residual_(x.clone())
+    _check(got, x, p, dev, f"M={M} C={C}")
+    want = x.double() + got.double()  # one rounding, against the separately rounded update
+    tol = (2.0**-7 if dtype == BF else 2.0**-22) * want.abs().max().item()
+    assert (res.double() - want).abs().max().item() <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, BF], ids=["fp32", "bf16"])
+def test_transition_few_rows_unaligned(dev, dtype):
+    print(f"[few rows] unaligned input {dtype}", flush=True)
+    m, p = _transition(dev, 384, 4, 3)
+    x = torch.randn(50, 384, generator=torch.Generator().manual_seed(1)).to(dev, dtype)
+    off = torch.empty(x.numel() + 1, dtype=dtype, device=dev)[1:].view(x.shape).copy_(x)
+    with torch.no_grad():
+        got = m.to(dtype)(off)
+    _check(got, x, p, dev, "unaligned")
+
+
+@pytest.mark.parametrize("M,K,N", [(3, 64, 16), (70, 160, 48), (300, 384, 1536), (5300, 64, 1536)])
+def test_layernorm_linear_bias(dev, M, K, N):
+    print(f"[few rows] LN + linear with bias M={M} K={K} N={N}", flush=True)
+    g = torch.Generator().manual_seed(M)
+    x, W, b = torch.randn(M, K, generator=g), torch.randn(K, N, generator=g) / K**0.5, torch.randn(N, generator=g)
+    lw, lb = 1 + 0.1 * torch.randn(K, generator=g), 0.1 * torch.randn(K, generator=g)
+    m = fused.FusedLayerNormLinear(K, N, has_linear_bias=True)
+    with torch.no_grad():
+        got = m(*(t.to(dev) for t in (x, lw, lb, W, b)))
+    ref = torch.nn.functional.layer_norm(x.double(), (K,), lw.double(), lb.double()) @ W.double() + b.double()
+    assert_fp32_close(got.cpu(), ref, what=f"LN + linear M={M}")
