@@ -12,6 +12,7 @@
 //                    the transition, LN' reads the updated z (rounded to z's dtype first, as
 //                    the reference computes it from the stored residual stream).
 #include <algorithm>
+#include <type_traits>
 
 #include "capi.h"
 #include "common.h"
@@ -25,9 +26,9 @@ constexpr int kS2pHeads = 16;
 template <class TC>
 constexpr int tr_bm() { return sizeof(TC) == 2 ? 64 : 32; }
 
-template <class TZ, class TC>
+template <class TZ, class TC, int BM_>
 struct TrCfg {
-  static constexpr int BM = tr_bm<TC>();
+  static constexpr int BM = BM_;
   static constexpr int ALD = kC + lds_pad<TC>();
   static constexpr int A_BYTES = BM * ALD * (int)sizeof(TC);
   static constexpr int SLD = kC + 4;
@@ -61,13 +62,13 @@ PF_DEVICE void s2p_store(const TC* A, int ALD, const TC* __restrict__ Ws, float*
   }
 }
 
-template <class TZ, class TC, bool S2P>
+template <class TZ, class TC, bool S2P, int BM_>
 __global__ __launch_bounds__(256) void pair_transition_kernel(
     const TZ* __restrict__ x, TZ* __restrict__ out, const float* __restrict__ lnw, const float* __restrict__ lnb,
     float eps, const TC* __restrict__ W1, const TC* __restrict__ W2, long M, int accumulate,
     const float* __restrict__ s2p_w, const float* __restrict__ s2p_b, float s2p_eps, const TC* __restrict__ Ws2p,
     float* __restrict__ logits, long NN) {
-  using Cfg = TrCfg<TZ, TC>;
+  using Cfg = TrCfg<TZ, TC, BM_>;
   constexpr int BM = Cfg::BM, ALD = Cfg::ALD, SLD = Cfg::SLD;
   constexpr int NT = 256;
   constexpr int RB = BM / 16;
@@ -284,8 +285,8 @@ __global__ __launch_bounds__(512) void pair_transition32_kernel(
   }
 }
 
-// bf16 path, persistent and weight-streaming: one 8-wave block per CU (two waves per SIMD)
-// walks tiles of 256 positions, 32 per wave (one MFMA column tile). Per tile each wave
+// bf16 path, persistent and weight-streaming: one block per CU (eight waves, two per SIMD; four
+// when one round of smaller tiles covers the rows) walks tiles of 32 positions per wave (one MFMA column tile). Per tile each wave
 // normalises its positions straight into registers as the B operands of W1 (fp32
 // statistics; a position's 128 channels live in lanes l and l ^ 32). The hidden dim is
 // walked in eight chunks of 64 (a rows 64 c .., b rows 512 + 64 c ..): the chunk's W1 rows
@@ -303,21 +304,18 @@ struct TransWs {
   static constexpr int C = 128;
   static constexpr int HC = 64;                      // hidden units per chunk
   static constexpr int NCH = kHidden / HC;           // 8 chunks
-  static constexpr int NW = 8;                       // waves per block (two per SIMD)
-  static constexpr int NT = 64 * NW;
-  static constexpr int PW = 32;                      // positions per wave
-  static constexpr int BP = PW * NW;                 // positions per tile
+  static constexpr int PW = 32;                      // positions per wave; a tile is NW waves' worth
   static constexpr int W1_BYTES = 2 * HC * C * 2;    // 128 rows x 256 B
   static constexpr int W2_BYTES = C * HC * 2;        // 128 rows x 128 B
   static constexpr int STAGE = W1_BYTES + W2_BYTES;  // 48 KiB
   static constexpr int U_BYTES = PW * HC * 2;        // per wave
-  static constexpr int DMA1 = W1_BYTES / 1024 / NW;  // W1 direct loads per wave per chunk
-  static constexpr int DMA2 = W2_BYTES / 1024 / NW;  // W2 direct loads per wave per chunk
+  static constexpr int DMA1 = W1_BYTES / 1024;       // W1 direct loads per chunk (split over the waves)
+  static constexpr int DMA2 = W2_BYTES / 1024;       // W2 direct loads per chunk
   static constexpr int S2P_BYTES = 8 * 64 * 16;      // Ws2p A fragments [k-step][lane]
 };
 
-constexpr size_t tr_ws_lds_bytes() {
-  return 2 * (size_t)TransWs::STAGE + (size_t)TransWs::NW * TransWs::U_BYTES + TransWs::S2P_BYTES +
+constexpr size_t tr_ws_lds_bytes(int waves) {
+  return 2 * (size_t)TransWs::STAGE + (size_t)waves * TransWs::U_BYTES + TransWs::S2P_BYTES +
          4 * TransWs::C * sizeof(float);
 }
 
@@ -369,18 +367,18 @@ struct ZRow {
   }
 };
 
-template <class TZ, bool S2P>
-__global__ __launch_bounds__(TransWs::NT, 1) void pair_transition_ws_kernel(
+template <class TZ, bool S2P, int NW>
+__global__ __launch_bounds__(64 * NW, 1) void pair_transition_ws_kernel(
     const TZ* __restrict__ x, TZ* __restrict__ out, const float* __restrict__ lnw, const float* __restrict__ lnb,
     float eps, const bf16* __restrict__ W1, const bf16* __restrict__ W2, long M, int accumulate,
     const float* __restrict__ s2p_w, const float* __restrict__ s2p_b, float s2p_eps, const bf16* __restrict__ Ws2p,
     float* __restrict__ logits, long NN) {
   using Cfg = TransWs;
-  constexpr int C = Cfg::C, HC = Cfg::HC, NCH = Cfg::NCH, PW = Cfg::PW, BP = Cfg::BP;
-  __shared__ __attribute__((aligned(16))) char smem[tr_ws_lds_bytes()];
+  constexpr int C = Cfg::C, HC = Cfg::HC, NCH = Cfg::NCH, PW = Cfg::PW, BP = PW * NW, NT = 64 * NW;
+  __shared__ __attribute__((aligned(16))) char smem[tr_ws_lds_bytes(NW)];
   char* stage0 = smem;                                      // [2][STAGE]
   char* ubase = smem + 2 * Cfg::STAGE;                      // [NW][U_BYTES]
-  char* s2pa = ubase + Cfg::NW * Cfg::U_BYTES;              // [8][64] x 16 B
+  char* s2pa = ubase + NW * Cfg::U_BYTES;              // [8][64] x 16 B
   float* lnp = reinterpret_cast<float*>(s2pa + Cfg::S2P_BYTES);  // lnw | lnb | s2p_w | s2p_b
 
   const int w = wave_id();
@@ -389,7 +387,7 @@ __global__ __launch_bounds__(TransWs::NT, 1) void pair_transition_ws_kernel(
   char* ub = ubase + w * Cfg::U_BYTES;
   const long ntiles = (M + BP - 1) / BP;
 
-  for (int i = threadIdx.x; i < C; i += Cfg::NT) {
+  for (int i = threadIdx.x; i < C; i += NT) {
     lnp[i] = lnw[i];
     lnp[C + i] = lnb[i];
     if (S2P) {
@@ -397,14 +395,17 @@ __global__ __launch_bounds__(TransWs::NT, 1) void pair_transition_ws_kernel(
       lnp[3 * C + i] = s2p_b[i];
     }
   }
-  if (S2P && w == 0) {
+  if (S2P) {
     // k-step ks takes channels 16 ks + 8 hf + e (the epilogue's lane-pair-swapped order);
-    // rows >= 16 are zero.
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
+    // rows >= 16 are zero. One 16-byte load per lane and step, unconditional (Ws2p may be on any
+    // 2-byte boundary): element loads under a condition made eight round trips before the
+    // first tile.
+    typedef __attribute__((ext_vector_type(8), aligned(2))) __bf16 bf16x8_u;
+    for (int ks = w; ks < 8; ks += NW) {
+      const bf16x8_u raw = *reinterpret_cast<const bf16x8_u*>(Ws2p + (lq & 15) * C + 16 * ks + 8 * hf);
       bf16x8 a;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) a[e] = lq < kS2pHeads ? Ws2p[lq * C + 16 * ks + 8 * hf + e] : (bf16)0.f;
+      for (int e = 0; e < 8; ++e) a[e] = lq < kS2pHeads ? raw[e] : (bf16)0.f;
       *reinterpret_cast<bf16x8*>(s2pa + (ks * 64 + l) * 16) = a;
     }
   }
@@ -416,16 +417,18 @@ __global__ __launch_bounds__(TransWs::NT, 1) void pair_transition_ws_kernel(
     const int c = (int)(g % NCH);
     char* st = stage0 + (g & 1) * Cfg::STAGE;
 #pragma unroll
-    for (int t = 0; t < Cfg::DMA1; ++t) {
-      const int ins = w * Cfg::DMA1 + t;  // 4 LDS rows of 256 B per instruction
+    for (int t = 0; t < (Cfg::DMA1 + NW - 1) / NW; ++t) {
+      const int ins = Cfg::DMA1 % NW == 0 ? w * (Cfg::DMA1 / NW) + t : w + NW * t;  // 4 rows of 256 B each
+      if (Cfg::DMA1 % NW != 0 && ins >= Cfg::DMA1) break;
       const int row = 4 * ins + (l >> 4);
       const int lc = (l & 15) ^ swz(row, 256);  // logical chunk this lane fetches
       const int grow = row < HC ? HC * c + row : kHidden + HC * c + (row - HC);
       buf_load_lds16(r1, st + ins * 1024, (grow * C + 8 * lc) * 2, 0);
     }
 #pragma unroll
-    for (int t = 0; t < Cfg::DMA2; ++t) {
-      const int ins = w * Cfg::DMA2 + t;  // 8 LDS rows of 128 B per instruction
+    for (int t = 0; t < (Cfg::DMA2 + NW - 1) / NW; ++t) {
+      const int ins = Cfg::DMA2 % NW == 0 ? w * (Cfg::DMA2 / NW) + t : w + NW * t;  // 8 rows of 128 B each
+      if (Cfg::DMA2 % NW != 0 && ins >= Cfg::DMA2) break;
       const int row = 8 * ins + (l >> 3);
       const int lc = (l & 7) ^ swz(row, 128);
       buf_load_lds16(r2, st + Cfg::W1_BYTES + ins * 1024, (row * kHidden + HC * c + 8 * lc) * 2, 0);
@@ -927,29 +930,49 @@ int transition_launch(const void* x, const float* lnw, const float* lnb, float e
                       const void* ws2p, float* logits, long NN, hipStream_t s) {
   pf::KernelTimer timer("pair_transition", s);
   if constexpr (sizeof(TC) == 2) {
-    const long ntiles = (M + TransWs::BP - 1) / TransWs::BP;
-    const unsigned nblk = (unsigned)std::min<long>(ntiles, pf::cu_count());
-    if (logits)
-      pair_transition_ws_kernel<TZ, true><<<nblk, TransWs::NT, 0, s>>>(
-          (const TZ*)x, (TZ*)out, lnw, lnb, eps, (const bf16*)w1, (const bf16*)w2, M, accumulate, s2p_w, s2p_b,
-          s2p_eps, (const bf16*)ws2p, logits, NN);
+    auto launch = [&](auto waves) {
+      constexpr int NW = decltype(waves)::value;
+      const long ntiles = (M + 32 * NW - 1) / (32 * NW);
+      const unsigned nblk = (unsigned)std::min<long>(ntiles, pf::cu_count());
+      if (logits)
+        pair_transition_ws_kernel<TZ, true, NW><<<nblk, 64 * NW, 0, s>>>(
+            (const TZ*)x, (TZ*)out, lnw, lnb, eps, (const bf16*)w1, (const bf16*)w2, M, accumulate, s2p_w, s2p_b,
+            s2p_eps, (const bf16*)ws2p, logits, NN);
+      else
+        pair_transition_ws_kernel<TZ, false, NW><<<nblk, 64 * NW, 0, s>>>(
+            (const TZ*)x, (TZ*)out, lnw, lnb, eps, (const bf16*)w1, (const bf16*)w2, M, accumulate, nullptr, nullptr,
+            0.f, nullptr, nullptr, NN);
+    };
+    // Four-wave tiles of 128 positions while they fit the CUs in one round, eight-wave tiles
+    // beyond (each wave does the same work in either, so results do not depend on it). bf16 with
+    // single_to_pair: N = 64 25 against 29 us, N = 181 28 against 32; N = 192, two rounds of four
+    // waves: 48 against 32. Six waves win only where three rounds of them come out even (N = 384
+    // fp32 stream: 104 against 111 us, bf16 90 against 89): not kept.
+    if (M <= 128L * pf::cu_count())
+      launch(std::integral_constant<int, 4>{});
     else
-      pair_transition_ws_kernel<TZ, false><<<nblk, TransWs::NT, 0, s>>>(
-          (const TZ*)x, (TZ*)out, lnw, lnb, eps, (const bf16*)w1, (const bf16*)w2, M, accumulate, nullptr, nullptr,
-          0.f, nullptr, nullptr, NN);
+      launch(std::integral_constant<int, 8>{});
     timer.stop();
     return pf::check_launch("pair_transition");
   }
-  constexpr int BM = tr_bm<TC>();
-  dim3 grid((unsigned)((M + BM - 1) / BM));
-  if (logits)
-    pair_transition_kernel<TZ, TC, true><<<grid, 256, 0, s>>>((const TZ*)x, (TZ*)out, lnw, lnb, eps, (const TC*)w1,
-                                                             (const TC*)w2, M, accumulate, s2p_w, s2p_b, s2p_eps,
-                                                             (const TC*)ws2p, logits, NN);
+  auto launch = [&](auto rows) {
+    constexpr int BM = decltype(rows)::value;
+    const unsigned grid = (unsigned)((M + BM - 1) / BM);
+    if (logits)
+      pair_transition_kernel<TZ, TC, true, BM><<<grid, 256, 0, s>>>(
+          (const TZ*)x, (TZ*)out, lnw, lnb, eps, (const TC*)w1, (const TC*)w2, M, accumulate, s2p_w, s2p_b, s2p_eps,
+          (const TC*)ws2p, logits, NN);
+    else
+      pair_transition_kernel<TZ, TC, false, BM><<<grid, 256, 0, s>>>(
+          (const TZ*)x, (TZ*)out, lnw, lnb, eps, (const TC*)w1, (const TC*)w2, M, accumulate, nullptr, nullptr, 0.f,
+          nullptr, nullptr, NN);
+  };
+  // 16-row tiles while the CUs take them in one round: N = 64 with single_to_pair 42 -> 31 us; past
+  // that they read the weights from L2 twice as often for the same work.
+  if (M <= 16L * pf::cu_count())
+    launch(std::integral_constant<int, 16>{});
   else
-    pair_transition_kernel<TZ, TC, false><<<grid, 256, 0, s>>>((const TZ*)x, (TZ*)out, lnw, lnb, eps, (const TC*)w1,
-                                                              (const TC*)w2, M, accumulate, nullptr, nullptr, 0.f,
-                                                              nullptr, nullptr, NN);
+    launch(std::integral_constant<int, 32>{});
   timer.stop();
   return pf::check_launch("pair_transition");
 }
