@@ -182,7 +182,8 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the raw handle of torch.cuda.current_stream(t.device), without building the Stream object
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def require_device(name: str, *ts: torch.Tensor) -> None:

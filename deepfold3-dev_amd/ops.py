@@ -25,6 +25,7 @@ from .kernels import (
     MHR_HEAD_NORMS,
     MHR_ROUTER_KINDS,
     FusedTriMulFunction,
+    block_order,
     cast_weight,
     gemm_dtype_for,
     layer_norm_for_gemm,
@@ -134,12 +135,12 @@ class _TriangleMulBase(nn.Module):
         out_proj."""
         nl = self.norm_left
         x = layer_norm_for_gemm(z, nl.weight, nl.bias, nl.eps)
-        order = self._block_order.to(z.device)
         w_out = self.out_proj.weight if scale == 1.0 else self.out_proj.weight * scale
         if self.router_stats_enabled and self.use_router:
             self._record_router_stats(self._router_gates(z))
         return FusedTriMulFunction.apply(
-            x.contiguous(), mask, self.gate.weight[order], self.proj.weight[order], self.norm_center.weight,
+            x.contiguous(), mask, block_order(self.gate.weight, self._outgoing),
+            block_order(self.proj.weight, self._outgoing), self.norm_center.weight,
             self.norm_center.bias, w_out, self.out_gate.weight, self.norm_center.eps, self._outgoing,
             None if self.router is None else self.router.weight, self._mix_codes(),
         )  # fmt: skip

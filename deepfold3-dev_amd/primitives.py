@@ -54,7 +54,7 @@ class WeightCache:
 
     def get(self, params: list[torch.Tensor | None], dtype: torch.dtype, build, tag=None):
         slot = (dtype, tag)
-        key = tuple(None if p is None else (p.data_ptr(), p._version) for p in params)
+        key = [None if p is None else (p.data_ptr(), p._version) for p in params]
         hit = self._entries.get(slot)
         if hit is not None and hit[0] == key:
             return hit[1]

@@ -188,3 +188,16 @@ def test_split_chunk():
     assert kernels._split_chunk(768 * 768) == 4096
     assert kernels._split_chunk(190 * 190) == 3610
     assert kernels._split_chunk(32761) == 4096  # 181^2 = 32761: no divisor in range
+
+
+@pytest.mark.parametrize("outgoing", [True, False], ids=["out", "in"])
+def test_block_order_is_the_row_permutation(outgoing):
+    """``kernels.block_order`` against indexing by the module's row list, value and gradient."""
+    k, ops_ = mod("kernels"), mod("ops")
+    m = (ops_.TriangleMulOutgoing if outgoing else ops_.TriangleMulIncoming)(64)
+    w = torch.randn(128, 64, requires_grad=True)
+    g = torch.randn(128, 64)
+    want = w[m._block_order]
+    got = k.block_order(w, outgoing)
+    assert torch.equal(got, want) and got.is_contiguous()
+    assert torch.equal(torch.autograd.grad(got, w, g)[0], torch.autograd.grad(want, w, g)[0])
