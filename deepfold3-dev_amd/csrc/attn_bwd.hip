@@ -96,6 +96,23 @@ PF_DEVICE f32x4 bfrag_from_acc<float>(const f32x16& acc, int t) {
   return f32x4{acc[4 * t], acc[4 * t + 1], acc[4 * t + 2], acc[4 * t + 3]};
 }
 
+// Blocks reach the eight XCDs round-robin: renumbered, each XCD takes one contiguous run of
+// block numbers (the remainder past a multiple of eight keeps its number), so the blocks that
+// read the same lines meet in one L2 instead of filling eight. Measured at B = 1, N = S = 384,
+// H = 4 in bf16: dK / dV 203 -> 166 us, dQ 152 -> 141, bias gradient 151 -> 137.
+PF_DEVICE unsigned xcd_run(unsigned id, unsigned total) {
+  const unsigned per = total >> 3;
+  return id < per * 8 ? (id & 7) * per + (id >> 3) : id;
+}
+struct Block3 {
+  unsigned x, y, z;
+};
+PF_DEVICE Block3 xcd_block() {
+  const unsigned nx = gridDim.x, ny = gridDim.y;
+  const unsigned id = xcd_run((blockIdx.z * ny + blockIdx.y) * nx + blockIdx.x, nx * ny * gridDim.z);
+  return {id % nx, id / nx % ny, id / (nx * ny)};
+}
+
 // Accumulator row r of lane half h.
 PF_DEVICE int acc_row(int r, int h) { return 8 * (r >> 2) + 4 * h + (r & 3); }
 
@@ -258,24 +275,25 @@ __global__ __launch_bounds__(kNT, sizeof(TC) == 2 ? 3 : 2) void attn_bwd_dq_kern
   __shared__ __attribute__((aligned(16))) float bstage[2][kRows * BLD];
   __shared__ __attribute__((aligned(16))) float mstage[2][kLines * 32];  // [line][key]
 
-  const int bh = blockIdx.z;
+  const Block3 blk = xcd_block();  // the query tiles of one line group in a row
+  const int bh = blk.z;
   const int b = bh / H;
   const int hd = bh % H;
   const int w = wave_id();
   const int l = lane_id();
   const int hh = l >> 5;
   const int c = l & 31;
-  const int s = blockIdx.y * kLines + w;
+  const int s = blk.y * kLines + w;
   const bool active = s < S;  // inactive waves mirror the group's first line and skip the math
-  const long sl = active ? s : (int)blockIdx.y * kLines;  // this wave's line (or the mirrored one)
+  const long sl = active ? s : (int)blk.y * kLines;  // this wave's line (or the mirrored one)
   const long bs = (long)b * S + sl;
   const size_t line = (size_t)bs * H + hd;
   const TC* Vl = V + line_offset(sx, b, sl, hd);
   const float off = kOff ? lineoff[bs] : 0.f;  // eager rule: this line's logit offset
   // line whose key mask thread t < 128 stages (the four lines of the group, clamped)
-  const float* m2s = mask2 + ((long)b * S + min((int)blockIdx.y * kLines + (int)(threadIdx.x >> 5), S - 1)) * Np;
+  const float* m2s = mask2 + ((long)b * S + min((int)blk.y * kLines + (int)(threadIdx.x >> 5), S - 1)) * Np;
   const float* b2l = bias2 + (size_t)bh * Np * Np;
-  const int q0 = blockIdx.x * kRows;
+  const int q0 = blk.x * kRows;
   const float sl2 = scale * kLog2e;
   const int nkt = (N + 31) / 32;
 
@@ -563,27 +581,28 @@ __global__ __launch_bounds__(kNT, sizeof(TC) == 2 ? 3 : 2) void attn_bwd_dkdv_ke
   __shared__ __attribute__((aligned(16))) float bstage[2][kRows * BLD];
   __shared__ __attribute__((aligned(16))) f32x4 sstage[2][kLines * 32];
 
-  const int bh = blockIdx.z;
+  const Block3 blk = xcd_block();  // the key tiles of one line group in a row
+  const int bh = blk.z;
   const int b = bh / H;
   const int hd = bh % H;
   const int w = wave_id();
   const int l = lane_id();
   const int hh = l >> 5;
   const int c = l & 31;
-  const int s = blockIdx.y * kLines + w;
+  const int s = blk.y * kLines + w;
   const bool active = s < S;
-  const long sl = active ? s : (int)blockIdx.y * kLines;
+  const long sl = active ? s : (int)blk.y * kLines;
   const long bs = (long)b * S + sl;
   const size_t line = (size_t)bs * H + hd;
   const long lo = line_offset(sg, b, sl, hd);  // this line's dK / dV rows
   const float off = kOff ? lineoff[bs] : 0.f;  // eager rule: this line's logit offset
   const float* b2l = bias2 + (size_t)bh * Np * Np;
-  const int kb0 = blockIdx.x * kRows;
+  const int kb0 = blk.x * kRows;
   const float sl2 = scale * kLog2e;
   const int nqt = (N + 31) / 32;
   // line whose statistics thread t < 128 stages (the four lines of the group, clamped)
   const int sw = threadIdx.x >> 5;
-  const size_t sline = ((size_t)b * S + min((int)blockIdx.y * kLines + sw, S - 1)) * H + hd;
+  const size_t sline = ((size_t)b * S + min((int)blk.y * kLines + sw, S - 1)) * H + hd;
 
   typename M::Frag kf[kSub][STEPS], vf[kSub][STEPS];
   float mk2[kSub];
@@ -732,16 +751,17 @@ __global__ __launch_bounds__(kNT, 3) void attn_bwd_db_kernel(const TC* __restric
                                                           const float* __restrict__ lineoff) {
   using M = Mfma<TC>;
   constexpr int STEPS = kBD / M::K32;
-  const int bh = blockIdx.z / groups;
-  const int grp = blockIdx.z % groups;
+  const Block3 blk = xcd_block();  // the tiles of one line group in a row
+  const int bh = blk.z / groups;
+  const int grp = blk.z % groups;
   const int b = bh / H;
   const int hd = bh % H;
   const int w = wave_id();
   const int l = lane_id();
   const int hh = l >> 5;
   const int c = l & 31;
-  const int q = blockIdx.x * 64 + (w & 1) * 32 + c;
-  const int k0 = blockIdx.y * 64 + (w >> 1) * 32;
+  const int q = blk.x * 64 + (w & 1) * 32 + c;
+  const int k0 = blk.y * 64 + (w >> 1) * 32;
   const float sl2 = scale * kLog2e;
   const int s_begin = (int)((long)S * grp / groups);
   const int s_end = (int)((long)S * (grp + 1) / groups);
