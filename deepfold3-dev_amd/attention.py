@@ -81,34 +81,34 @@ class GridSelfAttention(nn.Module):
 
     def _forward_grad(self, z: torch.Tensor, mask: torch.Tensor, scale: float) -> torch.Tensor:
         """Training path, as the reference's fused-attention branch (``attention.py:211-257``):
-        LayerNorm, pair bias and q/k/v/g projections in autograd, the HIP flash attention with
-        its backward (the kernel's masked-row rule), gate and output projection in autograd.
-        With 4 heads the attention (``fused._GridAttnCore``) reads the token-major projection
-        and writes O and the gradients in that order through strides; other head counts go
-        through the kernel-layout ``fused._EvoformerAttention``. Head dimension 32; ``scale`` on
-        out_proj."""
+        LayerNorm, pair bias and q/k/v/g projections, the HIP flash attention with its backward
+        (the kernel's masked-row rule), gate and output projection. With 4 heads the projections
+        are one node (``kernels.grid_projection``) and the attention with its gate
+        (``fused._GridAttnCore``) reads the token-major projection and writes the gated O and
+        the gradients in that order through strides; other head counts go through the
+        kernel-layout ``fused._EvoformerAttention``. Head dimension 32; ``scale`` on out_proj."""
         from .fused import _EvoformerAttention, _GridAttnCore
 
         B, N, _, C = z.shape
         H, D = self.num_heads, self.head_dim
         if D != 32:
             raise NotActive("GridSelfAttention", f"head dim {D}: the differentiable attention is built for 32")
-        from .kernels import layer_norm_for_gemm, token_linear
+        from .kernels import grid_projection, layer_norm_for_gemm, token_linear
 
         zn = layer_norm_for_gemm(z, self.norm.weight, self.norm.bias, self.norm.eps)
-        pb = token_linear(zn, self.pair_bias.weight).permute(0, 3, 1, 2)  # [B, H, N, N], un-transposed z
-        pb = pb.to(torch.float32, memory_format=torch.contiguous_format)
         line_mask = mask.transpose(1, 2) if self.transpose else mask  # [B, lines, keys]
         res_mask = torch.where(line_mask > 0.5, 0.0, -1e9).contiguous()
         w_out = self.out_proj.weight if scale == 1.0 else self.out_proj.weight * scale
-        g = torch.sigmoid(token_linear(zn, self.to_g.weight))
         if H == 4:
-            # q, k, v in one product over the un-transposed tokens; the attention reads them and
-            # writes O (and, backward, the gradients) in that token order through strides
-            w_qkv = torch.cat([self.to_q.weight, self.to_k.weight, self.to_v.weight])
-            qkv = token_linear(zn, w_qkv).view(B, N, N, 3, H, D)
-            o = _GridAttnCore.apply(qkv, res_mask, pb, self.transpose)
-            return token_linear(o.view(B, N, N, H * D) * g, w_out)
+            # q, k, v, g in one product over the un-transposed tokens; the attention reads them
+            # and writes the gated O (and, backward, the gradients) in that token order through strides
+            w = torch.cat([self.to_q.weight, self.to_k.weight, self.to_v.weight, self.to_g.weight])
+            proj, pb = grid_projection(zn, w, self.pair_bias.weight)  # pb [B, H, N, N], un-transposed z
+            o = _GridAttnCore.apply(proj.view(B, N, N, 4, H, D), res_mask, pb, self.transpose)
+            return token_linear(o.view(B, N, N, H * D), w_out)
+        pb = token_linear(zn, self.pair_bias.weight).permute(0, 3, 1, 2)  # [B, H, N, N], un-transposed z
+        pb = pb.to(torch.float32, memory_format=torch.contiguous_format)
+        g = torch.sigmoid(token_linear(zn, self.to_g.weight))
         # other head counts: the kernel-layout op with its head groups
         w_qkv = torch.cat([self.to_q.weight, self.to_k.weight, self.to_v.weight])
         y = token_linear(zn, w_qkv).view(B, N, N, 3, H, D).unbind(3)  # backward: one stack

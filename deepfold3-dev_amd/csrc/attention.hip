@@ -1584,57 +1584,64 @@ __global__ __launch_bounds__(256) void mask_outer_check_kernel(const float* __re
 // size). In fp32, Q is pre-scaled by d^-1/2 log2 e (one fp32 rounding) and the bias and mask
 // are stored times log2 e, which keeps large biases at their own fp32 precision.
 // -inf mask entries become -1e9.
+//
+// One block packs 64 keys (two key blocks) of one (b, s, h): 16-byte loads and stores
+// throughout, V through LDS into Vt[d][slot] (bf16: the key-block tile). Bytes bound it: at
+// 384 lines x 384 keys x 4 heads in bf16 the three operands take 51 us (their bytes: 44); Q and K in one
+// kernel and V in another, with 2-byte V accesses, took 66 us.
 template <class TC>
-__global__ __launch_bounds__(256) void evo_pack_qk_kernel(const TC* __restrict__ q, const TC* __restrict__ k,
-                                                          TC* __restrict__ Qw, TC* __restrict__ Kw, int S, int N,
-                                                          int Np, float qscale, Strides4 sx) {
+__global__ __launch_bounds__(256) void evo_pack_qkv_kernel(const TC* __restrict__ q, const TC* __restrict__ k,
+                                                           const TC* __restrict__ v, TC* __restrict__ Qw,
+                                                           TC* __restrict__ Kw, TC* __restrict__ Vt, int S, int N,
+                                                           int Np, float qscale, Strides4 sx) {
   constexpr int VEC = 16 / sizeof(TC);
-  constexpr int CPT = kHeadDim / VEC;  // chunks per token
-  const size_t bsh = blockIdx.y;       // (b, s, h) flattened
-  const int idx = blockIdx.x * 256 + threadIdx.x;
-  if (idx >= Np * CPT) return;
-  const int t = idx / CPT;
-  const int d0 = (idx % CPT) * VEC;
-  float vq[VEC], vk[VEC];
-  if (t < N) {
-    const long off = (long)(bsh / ((size_t)S * kHeads)) * sx.b + (long)((bsh / kHeads) % S) * sx.s +
-                     (long)(bsh % kHeads) * sx.h + (long)t * sx.n + d0;
-    load16<TC>(q + off, vq);
-    load16<TC>(k + off, vk);
+  constexpr int CPT = kHeadDim / VEC;  // pieces per token
+  constexpr int R = 64;
+  constexpr int LD = kHeadDim + VEC;
+  __shared__ __attribute__((aligned(16))) TC tile[R * LD];
+  const size_t bsh = blockIdx.y;  // (b, s, h) flattened
+  const int k0 = blockIdx.x * R;
+  const long line = (long)(bsh / ((size_t)S * kHeads)) * sx.b + (long)((bsh / kHeads) % S) * sx.s +
+                    (long)(bsh % kHeads) * sx.h;
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) vq[e] *= qscale;
-  } else {
+  for (int i = threadIdx.x; i < R * CPT; i += 256) {
+    const int t = k0 + i / CPT;
+    const int d0 = (i % CPT) * VEC;
+    float vq[VEC];
+    u32x4 vk = {0u, 0u, 0u, 0u}, vv = {0u, 0u, 0u, 0u};
+    if (t < N) {
+      const long off = line + (long)t * sx.n + d0;
+      load16<TC>(q + off, vq);
+      vk = *reinterpret_cast<const u32x4*>(k + off);
+      vv = *reinterpret_cast<const u32x4*>(v + off);
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) vq[e] = vk[e] = 0.f;
-  }
-  store_vec<TC, VEC>(Qw + (bsh * Np + t) * kHeadDim + d0, vq);
-  if constexpr (sizeof(TC) == 2)  // key-block tiles (kv_chunk)
-    store_vec<TC, VEC>(Kw + (bsh * Np + (t & ~31)) * kHeadDim + 8 * kv_chunk(t & 31, d0 / 8), vk);
-  else
-    store_vec<TC, VEC>(Kw + (bsh * Np + t) * kHeadDim + d0, vk);
-}
-
-// One block per (32-key block, b s h): V[t][d] -> Vt[d][slot] (bf16: the key-block tile).
-template <class TC>
-__global__ __launch_bounds__(256) void evo_pack_v_kernel(const TC* __restrict__ v, TC* __restrict__ Vt, int S,
-                                                         int N, int Np, Strides4 sx) {
-  __shared__ float tile[32][kHeadDim + 1];
-  const size_t bsh = blockIdx.y;
-  const int k0 = blockIdx.x * 32;
-  const TC* vl = v + (long)(bsh / ((size_t)S * kHeads)) * sx.b + (long)((bsh / kHeads) % S) * sx.s +
-                 (long)(bsh % kHeads) * sx.h;
-  for (int i = threadIdx.x; i < 32 * kHeadDim; i += 256) {
-    const int t = i / kHeadDim, d = i % kHeadDim;
-    tile[t][d] = (k0 + t < N) ? to_f32(vl[(long)(k0 + t) * sx.n + d]) : 0.f;
+      for (int e = 0; e < VEC; ++e) vq[e] *= qscale;
+    } else {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) vq[e] = 0.f;
+    }
+    store_vec<TC, VEC>(Qw + (bsh * Np + t) * kHeadDim + d0, vq);
+    if constexpr (sizeof(TC) == 2)  // key-block tiles (kv_chunk)
+      *reinterpret_cast<u32x4*>(Kw + (bsh * Np + (t & ~31)) * kHeadDim + 8 * kv_chunk(t & 31, d0 / 8)) = vk;
+    else
+      *reinterpret_cast<u32x4*>(Kw + (bsh * Np + t) * kHeadDim + d0) = vk;
+    *reinterpret_cast<u32x4*>(tile + (i / CPT) * LD + d0) = vv;
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < 32 * kHeadDim; i += 256) {
-    const int d = i / 32, slot = i % 32;
-    const TC v = from_f32<TC>(tile[slot_key(slot)][d]);
+#pragma unroll
+  for (int i = threadIdx.x; i < R * CPT; i += 256) {
+    // piece i: VEC consecutive slots of dimension d
+    const int d = sizeof(TC) == 2 ? i % kHeadDim : i / (R / VEC);
+    const int s0 = (sizeof(TC) == 2 ? i / kHeadDim : i % (R / VEC)) * VEC;
+    TC e[VEC];
+#pragma unroll
+    for (int u = 0; u < VEC; ++u) e[u] = tile[((s0 & ~31) + slot_key((s0 & 31) + u)) * LD + d];
+    u32x4 p;
+    __builtin_memcpy(&p, e, 16);
     if constexpr (sizeof(TC) == 2)
-      Vt[(bsh * Np + k0) * kHeadDim + 8 * kv_chunk(d, slot / 8) + slot % 8] = v;
+      *reinterpret_cast<u32x4*>(Vt + (bsh * Np + k0 + (s0 & ~31)) * kHeadDim + 8 * kv_chunk(d, (s0 & 31) / 8)) = p;
     else
-      Vt[(bsh * kHeadDim + d) * Np + k0 + slot] = v;
+      *reinterpret_cast<u32x4*>(Vt + (bsh * kHeadDim + d) * Np + k0 + s0) = p;
   }
 }
 
@@ -1712,10 +1719,8 @@ int evo_attn_launch(const void* q, const void* k, const void* v, const float* re
   const float bscale = kPost ? 1.f / softmax_scale : kLog2e;
   const float post = softmax_scale * kLog2e;
   const unsigned bsh = (unsigned)(B * S * kHeads);
-  constexpr int VEC = 16 / sizeof(TC);
-  evo_pack_qk_kernel<TC><<<dim3((Np * (kHeadDim / VEC) + 255) / 256, bsh), 256, 0, s>>>(
-      (const TC*)q, (const TC*)k, Qw, Kw, S, N, Np, qscale, sx);
-  evo_pack_v_kernel<TC><<<dim3(Np / 32, bsh), 256, 0, s>>>((const TC*)v, Vw, S, N, Np, sx);
+  evo_pack_qkv_kernel<TC><<<dim3(Np / 64, bsh), 256, 0, s>>>((const TC*)q, (const TC*)k, (const TC*)v, Qw, Kw, Vw, S,
+                                                             N, Np, qscale, sx);
   evo_pack_bias_kernel<<<dim3((unsigned)(((long)Np * Np + 255) / 256), B * kHeads), 256, 0, s>>>(pair_bias, PBw,
                                                                                                    N, Np, bscale);
   evo_pack_mask_kernel<<<dim3((Np + 255) / 256, B * S), 256, 0, s>>>(res_mask, MAw, N, Np, bscale);

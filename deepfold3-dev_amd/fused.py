@@ -146,6 +146,10 @@ class _GridAttnCore(torch.autograd.Function):
     so nothing is permuted or copied around them. The kernel's masked-line rule (a line whose
     keys are all masked outputs 0). H = 4, D = 32.
 
+    With qkv ``[B, N, N, 4, H, D]`` the fourth part is the output gate's g: returns
+    ``O * sigmoid(g)``, and the backward forms dO and dg in one pass (``pf_grid_gate_fwd`` /
+    ``pf_grid_gate_bwd``), dg into its part of the one gradient.
+
     With ``use_lse`` (the default) the forward also writes each row's log-sum-exp and the
     backward's dQ kernel takes it in place of its own pass over the keys for the row maximum
     (``pf_evo_attn_bwd_strided``'s ``lse``; the reference saves softmax_lse the same way,
@@ -155,8 +159,8 @@ class _GridAttnCore(torch.autograd.Function):
 
     @staticmethod
     def _layout(qkv, transpose):
-        B, N1, N2, _, H, D = qkv.shape
-        tok = 3 * H * D
+        B, N1, N2, parts, H, D = qkv.shape
+        tok = parts * H * D
         if transpose:  # lines j, keys i
             sx = (N1 * N2 * tok, tok, D, N2 * tok)
             so = (N1 * N2 * H * D, H * D, D, N2 * H * D)
@@ -189,13 +193,21 @@ class _GridAttnCore(torch.autograd.Function):
             ws.data_ptr(), ws_bytes, _lib.stream_of(qkv),
         )  # fmt: skip
         _lib.note_redo("pf_evo_attn_redo_flags", ws, B, S, H, N, D, code)
-        ctx.save_for_backward(qkv, rm, pb, lse)
         ctx.transpose = bool(transpose)
-        return out
+        if qkv.shape[3] == 3:
+            ctx.save_for_backward(qkv, rm, pb, lse)
+            return out
+        ctx.save_for_backward(qkv, rm, pb, lse, out)
+        gated = torch.empty_like(out)
+        _lib.call(
+            "pf_grid_gate_fwd", out.data_ptr(), base + 3 * H * D * es, 4 * H * D, code, gated.data_ptr(), B * S * N,
+            H * D, _lib.stream_of(qkv),
+        )  # fmt: skip
+        return gated
 
     @staticmethod
     def backward(ctx, dO):
-        qkv, rm, pb, lse = ctx.saved_tensors
+        qkv, rm, pb, lse, *gate_o = ctx.saved_tensors
         B, S, H, N, D, sx, so = _GridAttnCore._layout(qkv, ctx.transpose)
         code = _lib.dtype_code(qkv.dtype)
         dO = dO.to(qkv.dtype).contiguous()
@@ -207,6 +219,12 @@ class _GridAttnCore(torch.autograd.Function):
         base, gbase = qkv.data_ptr(), dqkv.data_ptr()
         ax, px = _strides(*sx)
         ao, po = _strides(*so)
+        if gate_o:
+            dout, dO = dO, torch.empty_like(dO)
+            _lib.call(
+                "pf_grid_gate_bwd", dout.data_ptr(), gate_o[0].data_ptr(), base + 3 * H * D * es, 4 * H * D, code,
+                dO.data_ptr(), gbase + 3 * H * D * es, 4 * H * D, B * S * N, H * D, _lib.stream_of(qkv),
+            )  # fmt: skip
         kernel_census.record("GridSelfAttention.backward", "hip_evo_attn_bwd_strided")
         _lib.call(
             "pf_evo_attn_bwd_strided", base, base + H * D * es, base + 2 * H * D * es, px, rm.data_ptr(),

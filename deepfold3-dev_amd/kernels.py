@@ -504,6 +504,61 @@ def token_linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         return _TokenLinear.apply(x.contiguous(), weight)
 
 
+class _GridProjection(torch.autograd.Function):
+    """The projections of the grid attention's training path in one node: ``apply(x, w, w_bias)``
+    with x ``[B, N, N, 128]``, w ``[512, 128]`` (q | k | v | g rows) and w_bias ``[4, 128]`` of x's
+    dtype returns ``x w^T`` and the pair bias ``x w_bias^T`` as fp32 ``[B, 4, N, N]``. One product
+    over the four stacked projections each way (the input's gradient takes the bias's part as
+    its accumulator, so no gradient is added in a pass of its own); the pair bias and its
+    backward on ``pf_grid_bias_fwd`` / ``pf_grid_bias_bwd``."""
+
+    @staticmethod
+    def forward(ctx, x, w, w_bias):
+        w, w_bias = w.contiguous(), w_bias.contiguous()
+        ctx.save_for_backward(x, w, w_bias)
+        B, N, _, C = x.shape
+        pb = torch.empty((B, w_bias.shape[0], N, N), dtype=torch.float32, device=x.device)
+        _lib.call(
+            "pf_grid_bias_fwd", x.data_ptr(), w_bias.data_ptr(), _lib.dtype_code(x.dtype), B, N, C, w_bias.shape[0],
+            pb.data_ptr(), _lib.stream_of(x),
+        )  # fmt: skip
+        return torch.nn.functional.linear(x, w), pb
+
+    @staticmethod
+    def backward(ctx, gy, gpb):
+        x, w, w_bias = ctx.saved_tensors
+        B, N, _, C = x.shape
+        H = w_bias.shape[0]
+        x2 = x.view(-1, C)
+        gy2 = gy.to(x.dtype).contiguous().view(-1, w.shape[0])
+        gx = torch.empty_like(x)
+        gwb = torch.empty((H, C), dtype=torch.float32, device=x.device)
+        ws_bytes = _lib.lib().pf_grid_bias_bwd_workspace_bytes(B, N, C, H)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+        gpb = gpb.to(torch.float32).contiguous()
+        _lib.call(
+            "pf_grid_bias_bwd", x.data_ptr(), w_bias.data_ptr(), gpb.data_ptr(), _lib.dtype_code(x.dtype), B, N, C, H,
+            gx.data_ptr(), gwb.data_ptr(), ws.data_ptr(), ws_bytes, _lib.stream_of(x),
+        )  # fmt: skip
+        gx.view(-1, C).addmm_(gy2, w)
+        gw = None
+        if ctx.needs_input_grad[1]:
+            gw = gy2.t() @ x2 if len(x2) < SPLIT_K_TOKENS else _weight_grad_tm(gy2, x2).to(w.dtype)
+        return gx, gw, gwb.to(w_bias.dtype)
+
+
+def grid_projection(x: torch.Tensor, weight: torch.Tensor, weight_bias: torch.Tensor) -> tuple:
+    """``(x weight^T, fp32 [B, H, N, N] of x weight_bias^T)`` for the grid attention's training
+    path (``_GridProjection``), operands cast as autocast would cast them for a linear."""
+    if torch.is_autocast_enabled("cuda"):
+        dt = torch.get_autocast_dtype("cuda")
+        x, weight, weight_bias = x.to(dt), weight.to(dt), weight_bias.to(dt)
+    if not x.dtype == weight.dtype == weight_bias.dtype:
+        raise RuntimeError(f"grid_projection: x {x.dtype}, weights {weight.dtype} and {weight_bias.dtype} differ")
+    with torch.autocast("cuda", enabled=False):
+        return _GridProjection.apply(x.contiguous(), weight, weight_bias)
+
+
 def block_order(w: torch.Tensor, outgoing: bool) -> torch.Tensor:
     """The interleaved a / b rows of a [2C, C] triangle projection in block order: rows ``0::2``
     then ``1::2`` (outgoing), swapped for incoming (``ops.py:285-288``). Views and one copy, so its

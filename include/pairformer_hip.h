@@ -420,6 +420,20 @@ int pf_evo_attn_bwd_strided(const void* q, const void* k, const void* v, const l
                             const float* lse, int B, int S, int H, int N, int D, int dtype, float softmax_scale,
                             void* dq, void* dk, void* dv, const long* grad_strides, float* dpair_bias,
                             void* workspace, size_t workspace_bytes, void* stream);
+/* The row operators around the strided attention in GridSelfAttention's training path
+ * (attention.py:211-257), C = 128 channels in H = 4 heads, all pointers 16-byte aligned.
+ * pf_grid_bias_fwd: out [B, H, N, N] fp32 = x w^T for x [B, N, N, C] and w [H, C] in dtype.
+ * pf_grid_bias_bwd: from dout [B, H, N, N] fp32, dx [B, N, N, C] in dtype and dw [H, C] fp32
+ * (summed in a fixed order).
+ * pf_grid_gate_fwd: out [M, C] = o sigmoid(g), o [M, C], g in rows of ldg elements.
+ * pf_grid_gate_bwd: d_o [M, C] and dg (rows of lddg elements) from dout [M, C], o and g. */
+int pf_grid_bias_fwd(const void* x, const void* w, int dtype, int B, int N, int C, int H, float* out, void* stream);
+size_t pf_grid_bias_bwd_workspace_bytes(int B, int N, int C, int H);
+int pf_grid_bias_bwd(const void* x, const void* w, const float* dout, int dtype, int B, int N, int C, int H, void* dx,
+                     float* dw, void* workspace, size_t workspace_bytes, void* stream);
+int pf_grid_gate_fwd(const void* o, const void* g, long ldg, int dtype, void* out, long M, int C, void* stream);
+int pf_grid_gate_bwd(const void* dout, const void* o, const void* g, long ldg, int dtype, void* d_o, void* dg,
+                     long lddg, long M, int C, void* stream);
 /* FusedPairBias(c, H)(z, ln_w, ln_b, proj_w, mask) (triton/fused_pair_bias.py:348-416):
  * z [B,N,N,C] -> out [B,H,N,N] in z's dtype; proj_w16 [16, C] fp32 (proj_w padded with zero
  * rows); mask [B,N] fp32 or NULL adds (1 - mask) * (-1e9) on the last axis. C = 128, H <= 16. */

@@ -1,0 +1,105 @@
+"""Row operators around the training path of the grid attention on a real MI355X: the pair-bias
+projection and the output gate with their backwards, against fp64 on the same operands."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tests._helpers import mod
+
+pytestmark = pytest.mark.gpu
+
+_lib = mod("_lib")
+kernels = mod("kernels")
+fused = mod("fused")
+
+C, H = 128, 4
+EPS = {torch.float32: 2.0**-23, torch.bfloat16: 2.0**-8}
+
+
+@pytest.fixture(scope="module")
+def dev():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    return torch.device("cuda:0")
+
+
+def _operands(dev, B, N, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+
+    def r(*shape, s=1.0):
+        return (torch.randn(*shape, generator=g) * s).to(dev, dtype)
+
+    return r(B, N, N, C), r(4 * C, C, s=C**-0.5), r(H, C, s=C**-0.5), r(B, N, N, 4 * C), g
+
+
+# 1 and 7: less than a tile of 64 tokens; 8: exactly one; 23: a remainder, tiles over a batch
+# boundary; 190: more tiles (565) than blocks of the backward, and the split weight gradient
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("B,N", [(1, 1), (1, 7), (1, 8), (3, 23), (1, 190)])
+def test_grid_projection_and_gradients(dev, B, N, dtype):
+    """Each result within its rounding to ``dtype`` plus an fp32 sum's worst case: n 2^-23 of the
+    sum of the terms' magnitudes (the split weight gradient's chunks round to ``dtype`` once)."""
+    x, w, wb, gy, g = _operands(dev, B, N, dtype, 40 + N)
+    gpb = torch.randn(B, H, N, N, generator=g).to(dev)
+    print(f"[grid projection] B={B} N={N} {dtype}", flush=True)
+    xr, wr, wbr = (t.clone().requires_grad_(True) for t in (x, w, wb))
+    y, pb = kernels.grid_projection(xr, wr, wbr)
+    torch.autograd.backward([y, pb], [gy, gpb])
+    x2, g2, p2 = x.double().view(-1, C), gy.double().view(-1, 4 * C), gpb.double().permute(0, 2, 3, 1).reshape(-1, H)
+    wd, wbd = w.double(), wb.double()
+    M, f32 = x2.shape[0], 2.0**-23
+
+    def check(what, got, want, mag, n, rounds):
+        bound = rounds * EPS[dtype] * mag + n * f32 * mag + 1e-30
+        worst = ((got.double() - want).abs() / bound).max().item()
+        print(f"  {what}: {worst:.3f} of the bound", flush=True)
+        assert worst <= 1.0, what
+
+    assert pb.dtype == torch.float32 and pb.shape == (B, H, N, N)
+    tok = pb.permute(0, 2, 3, 1).reshape(-1, H)
+    check("pair bias", tok, x2 @ wbd.t(), x2.abs() @ wbd.abs().t(), C, 0)
+    check("projection", y.view(-1, 4 * C), x2 @ wd.t(), x2.abs() @ wd.abs().t(), C, 1)
+    mag = g2.abs() @ wd.abs() + p2.abs() @ wbd.abs()
+    check("dx", xr.grad.view(-1, C), g2 @ wd + p2 @ wbd, mag, 4 * C + H, 2)
+    check("dw", wr.grad, g2.t() @ x2, g2.abs().t() @ x2.abs(), M, 2)
+    check("dw_bias", wbr.grad, p2.t() @ x2, p2.abs().t() @ x2.abs(), M, 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("transpose", [False, True], ids=["rows", "cols"])
+@pytest.mark.parametrize("N", [1, 33, 130])
+def test_gated_attention_is_attention_times_gate(dev, N, transpose, dtype):
+    """``fused._GridAttnCore`` with the gate's part against the three-part form and the gate in
+    fp32: the same dq, dk, dv and bias gradient for the same dO; the gated output and dg within
+    their rounding (and the hardware exponential's, 2^-20 relative)."""
+    B = 2
+    g = torch.Generator().manual_seed(70 + N)
+    p4 = (torch.randn(B, N, N, 4, H, 32, generator=g) * 0.5).to(dev, dtype)
+    keep = torch.rand(B, N, N, generator=g) < 0.85
+    rm = torch.where(keep, 0.0, -1e9).to(dev)
+    pb = torch.randn(B, H, N, N, generator=g).to(dev)
+    dout = torch.randn(B, N, N, H, 32, generator=g).to(dev, dtype)
+    print(f"[gated attention] N={N} transpose={transpose} {dtype}", flush=True)
+    x4, b4 = p4.clone().requires_grad_(True), pb.clone().requires_grad_(True)
+    y = fused._GridAttnCore.apply(x4, rm, b4, transpose)
+    y.backward(dout)
+    x3, b3 = p4[:, :, :, :3].contiguous().requires_grad_(True), pb.clone().requires_grad_(True)
+    o = fused._GridAttnCore.apply(x3, rm, b3, transpose)
+    sg = torch.sigmoid(p4[:, :, :, 3].double())
+    want = o.detach().double() * sg
+    tol = EPS[dtype] + 2.0**-20
+    assert ((y.detach().double() - want).abs() <= tol * want.abs() + 1e-30).all()
+    wg = dout.double() * o.detach().double() * sg * (1 - sg)
+    assert ((x4.grad[:, :, :, 3].double() - wg).abs() <= (tol + 2.0**-20) * wg.abs() + 1e-30).all()
+    # dO as the kernel rounds it, through the three-part form
+    dO, scratch = torch.empty_like(dout), torch.empty_like(p4)
+    _lib.call(
+        "pf_grid_gate_bwd", dout.data_ptr(), o.data_ptr(), p4.data_ptr() + 3 * C * p4.element_size(), 4 * C,
+        _lib.dtype_code(dtype), dO.data_ptr(), scratch.data_ptr(), 4 * C, B * N * N, C,
+        _lib.stream_of(p4),
+    )  # fmt: skip
+    assert ((dO.double() - dout.double() * sg).abs() <= tol * (dout.double() * sg).abs() + 1e-30).all()
+    o.backward(dO)
+    assert torch.equal(x4.grad[:, :, :, :3], x3.grad) and torch.equal(b4.grad, b3.grad)
