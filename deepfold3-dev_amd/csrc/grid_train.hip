@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256) void grid_bias_fwd_kernel(const TC* __restrict
 // dx[b][p][c] = sum_h dpb[b][h][p] w[h][c] and, per block, the partial dw[h][c] = sum_p
 // dpb[b][h][p] x[b][p][c]: one read of x, one write of dx, fp32 sums. Two library products
 // (K = 4 and, split over tokens, an output of 4 rows) with the copies between the two orders
-// take 95 us at 384 x 384 tokens in bf16, this kernel 19 us and its reduction GBDW us.
+// take 95 us at 384 x 384 tokens in bf16, this kernel 19 us and its reduction 5 us.
 template <class TC>
 __global__ __launch_bounds__(256) void grid_bias_bwd_kernel(const TC* __restrict__ x, const TC* __restrict__ w,
                                                             const float* __restrict__ dpb, TC* __restrict__ dx,
