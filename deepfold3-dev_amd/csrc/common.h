@@ -431,6 +431,37 @@ PF_DEVICE void zero_acc32(f32x16 (&acc)[MI][NJ]) {
 PF_DEVICE __amdgpu_buffer_rsrc_t buf_rsrc(const void* p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
+// Buffer accesses in registers. An offset past the resource's bytes reads 0 and writes nothing,
+// so a ragged tile needs no branch around its accesses: a load behind a branch is waited for
+// inside it (a row of conditional loads is a row of memory round trips), and with a store
+// behind a branch the compiler cannot count it, so the next wait for a load waits for every
+// store as well. The whole offset is in voff: the scalar offset is subtracted from the bound,
+// not added to the offset, when the hardware compares the two.
+PF_DEVICE u32x4 buf_load16(__amdgpu_buffer_rsrc_t r, int voff) {
+  return __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0);
+}
+PF_DEVICE void buf_store16(__amdgpu_buffer_rsrc_t r, u32x4 v, int voff) {
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, voff, 0, 0);
+}
+// One element as its bits (bf16: the low half).
+template <class T>
+PF_DEVICE unsigned buf_load_bits(__amdgpu_buffer_rsrc_t r, int voff) {
+  if constexpr (sizeof(T) == 2)
+    return __builtin_amdgcn_raw_buffer_load_b16(r, voff, 0, 0);
+  else
+    return __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0);
+}
+template <class T>
+PF_DEVICE float bits_to_f32(unsigned v) {
+  return __uint_as_float(sizeof(T) == 2 ? v << 16 : v);
+}
+template <class T>
+PF_DEVICE void buf_store_elem(__amdgpu_buffer_rsrc_t r, float v, int voff) {
+  if constexpr (sizeof(T) == 2)
+    __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, from_f32<bf16>(v)), r, voff, 0, 0);
+  else
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, voff, 0, 0);
+}
 // 16 bytes per lane from a buffer straight into LDS: lane l lands at lds + 16 l (the LDS
 // address is taken from the wave's first lane). The host compilation pass cannot type-check
 // this builtin; kernels only run on the device.

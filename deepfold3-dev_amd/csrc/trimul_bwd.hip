@@ -329,9 +329,18 @@ __global__ __launch_bounds__(vjp_nt<C>()) void trimul_output_vjp_kernel(
 // trimul_output_vjp_kernel, with one 512-thread block per CU walking 64-position tiles. Wave w
 // takes the output columns 16 w .. +16 of all four GEMMs (xln Wo^T, x Wog^T, gp Wo, gg Wog);
 // their B fragments (16x16x32 steps, lane: column l & 15, k = 32 s + 8 (l >> 4) ..) are rows of
-// Wo, Wog, Wo^T, Wog^T and stay in registers for the whole kernel. The LN_out affine gradients
-// accumulate per thread (channel tid & 127, positions 16 (tid >> 7) .. +16 of every tile) and
-// leave as one partial sum per block.
+// Wo, Wog, Wo^T, Wog^T and stay in registers for the whole kernel.
+//
+// Memory bounds it (nine operands, 340 MB at B = 1, N = 384) and one block per CU has no other
+// to hide a round trip, so nothing of a tile is waited for when it is asked for: the next
+// tile's X and x are loaded as soon as this tile's are in LDS, the next tile's g as soon as
+// this tile's is used, and every access of tokens is a buffer access without a branch. With
+// g loaded where it was used, behind its bounds test, the sixteen loads of a lane were sixteen
+// round trips a tile: 167 us then, 77 us now.
+//
+// The per-position passes give thread (position tid >> 3, part os = tid & 7) the channel pairs
+// 16 k + 2 os + {0, 1}: the 64 lanes of a read of X [c][p] touch distinct banks. Their LN_out
+// affine gradients accumulate per thread over its tiles and leave as one partial sum per block.
 struct OutputVjpWs {
   static constexpr int C = 128;
   static constexpr int BM = 64;
@@ -339,8 +348,7 @@ struct OutputVjpWs {
   static constexpr int XLD = BM + 8;  // X tile [c][p] (bf16)
   static constexpr int ALD = C + 8;   // xln / x, then gp / gg, [p][c] (bf16)
   static constexpr int SLD = C + 4;   // d(xln) [p][c] (fp32)
-  static constexpr int NQ = NT / BM;  // threads per position in the per-position passes
-  static constexpr int CPQ = C / NQ;
+  static constexpr int CPQ = 16;      // channels per thread in the per-position passes
 };
 
 // acc[rb] (rows 16 rb .., columns of this wave) += A [64][C] (LDS, k contiguous) W, W's B
@@ -365,15 +373,17 @@ __global__ __launch_bounds__(OutputVjpWs::NT) void trimul_output_vjp_ws_kernel(
     float* __restrict__ partial) {
   using Cfg = OutputVjpWs;
   constexpr int C = Cfg::C, BM = Cfg::BM, NT = Cfg::NT, XLD = Cfg::XLD, ALD = Cfg::ALD, SLD = Cfg::SLD;
-  constexpr int NQ = Cfg::NQ, CPQ = Cfg::CPQ;
+  constexpr int CPQ = Cfg::CPQ;
+  constexpr int ES = (int)sizeof(TZ);
+  constexpr int XV = 16 / ES;               // x elements per 16-byte load
+  constexpr int XL = BM * C / XV / NT;      // x loads per thread per tile
+  constexpr int PL = C * BM / 8 / NT;       // plane (bf16) loads per thread per tile
   constexpr int A_BYTES = BM * ALD * 2;
   constexpr int ST_BYTES = BM * SLD * 4;
   constexpr int R_BYTES = 2 * A_BYTES > ST_BYTES ? 2 * A_BYTES : ST_BYTES;
   __shared__ __attribute__((aligned(16))) bf16 Xs[C * XLD];  // X [c][p], later dX
   __shared__ __attribute__((aligned(16))) char rsm[R_BYTES];
-  __shared__ float s_mean[BM], s_rstd[BM];
-  __shared__ float s_lnw[C], s_lnb[C];
-  __shared__ float red[2][NT];
+  __shared__ __attribute__((aligned(16))) float s_lnw[C], s_lnb[C];
   bf16* A1 = reinterpret_cast<bf16*>(rsm);            // xln, then gp
   bf16* A2 = reinterpret_cast<bf16*>(rsm + A_BYTES);  // x, then gg
   float* stage = reinterpret_cast<float*>(rsm);       // d(xln), fp32
@@ -382,8 +392,8 @@ __global__ __launch_bounds__(OutputVjpWs::NT) void trimul_output_vjp_ws_kernel(
   const int w = wave_id();
   const int l = lane_id();
   const size_t pe = (size_t)Np * Np;
-  const int tpl = Np / BM;
-  const int ntiles = B * Np * tpl;  // every tile of the planes, padding included (< 2^31)
+  const int tpl = (N + BM - 1) / BM;
+  const int ntiles = B * N * tpl;  // tiles that hold tokens (< 2^31, checked at launch)
   const int G = gridDim.x;
   const int col = 16 * w + (l & 15);  // this lane's output column in all four GEMMs
 
@@ -396,75 +406,95 @@ __global__ __launch_bounds__(OutputVjpWs::NT) void trimul_output_vjp_ws_kernel(
     wot[st] = *reinterpret_cast<const bf16x8*>(WoT + (size_t)col * C + k);
     wogt[st] = *reinterpret_cast<const bf16x8*>(WogT + (size_t)col * C + k);
   }
-  const int pq = tid / NQ;
-  const int qq = tid % NQ;
   if (tid < C) {
     s_lnw[tid] = lnow[tid];
     s_lnb[tid] = lnob[tid];
   }
-  float pw = 0.f, pb = 0.f;  // LN_out affine partials of channel tid & 127
+  const int op = tid >> 3, os = tid & 7;
+  auto och = [&](int c) { return 16 * (c >> 1) + 2 * os + (c & 1); };
+  float pw[CPQ] = {}, pb[CPQ] = {};  // LN_out affine partials of this thread's channels
 
-  for (int tile = blockIdx.x; tile < ntiles; tile += G) {
-    const int b = tile / (Np * tpl);
-    const int rem = tile - b * (Np * tpl);
-    const int i = rem / tpl;
-    const int j0 = (rem - i * tpl) * BM;
-    const int nvalid = i < N ? max(0, min(BM, N - j0)) : 0;
-    const long tok0 = ((long)b * N + i) * N + j0;  // position p is token tok0 + p (p < nvalid)
-    if (nvalid == 0) {
-      // padding only: dX is zero there (the contraction's cotangent GEMMs read it)
-      bf16* Db = dX + (size_t)b * C * pe + (size_t)i * Np + j0;
+  // Tile -> plane row i, first position j0, tokens of the tile (consecutive from tok0).
+  struct Tile {
+    int b, i, j0, nvalid;
+    long tok0;
+  };
+  auto tile_at = [&](int tile) {
+    Tile t;
+    t.b = tile / (N * tpl);
+    const int rem = tile - t.b * (N * tpl);
+    t.i = rem / tpl;
+    t.j0 = (rem - t.i * tpl) * BM;
+    t.nvalid = min(BM, N - t.j0);
+    t.tok0 = ((long)t.b * N + t.i) * N + t.j0;
+    return t;
+  };
+  u32x4 Xr[PL], xr[XL];
+  unsigned gr[16];
+  const int poff = (tid / (BM / 8)) * XLD + 8 * (tid % (BM / 8));  // plane piece: channel tid / 8 (+ 64 q)
+  auto issue_x = [&](int tile) __attribute__((always_inline)) {
+    const Tile t = tile_at(tile);
+    const bf16* Xb = X + (size_t)t.b * C * pe + (size_t)t.i * Np + t.j0 + (size_t)(tid / (BM / 8)) * pe +
+                     8 * (tid % (BM / 8));
 #pragma unroll
-      for (int it = 0; it < C * BM / 8 / NT; ++it) {
-        const int idx = tid + it * NT;
-        *reinterpret_cast<u32x4*>(Db + (size_t)(idx / (BM / 8)) * pe + (idx % (BM / 8)) * 8) = u32x4{0u, 0u, 0u, 0u};
-      }
-      continue;  // block-uniform
-    }
+    for (int q = 0; q < PL; ++q) Xr[q] = *reinterpret_cast<const u32x4*>(Xb + (size_t)q * (NT / (BM / 8)) * pe);
+    const auto r = buf_rsrc(x + t.tok0 * C, t.nvalid * C * ES);
+#pragma unroll
+    for (int q = 0; q < XL; ++q) xr[q] = buf_load16(r, 16 * (tid + NT * q));
+  };
+  auto issue_g = [&](int tile) __attribute__((always_inline)) {
+    const Tile t = tile_at(tile);
+    const auto r = buf_rsrc(g + t.tok0 * C, t.nvalid * C * ES);
+    const int off = (4 * (l >> 4) * C + col) * ES;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) gr[q] = buf_load_bits<TZ>(r, off + (16 * (q >> 2) + (q & 3)) * C * ES);
+  };
 
-    // X tile, channel-major (rows of 64 contiguous positions per channel); x rows
-    {
-      const bf16* Xb = X + (size_t)b * C * pe + (size_t)i * Np + j0;
+  int tile = blockIdx.x;
+  if (tile < ntiles) {
+    issue_x(tile);
+    issue_g(tile);
+  }
+  for (; tile < ntiles; tile += G) {
+    const Tile t = tile_at(tile);
+    const int next = min(tile + G, ntiles - 1);
+    const unsigned row_bytes = t.nvalid * C * 2;  // the tile's rows of a bf16 operand
 #pragma unroll
-      for (int it = 0; it < C * BM / 8 / NT; ++it) {
-        const int idx = tid + it * NT;
-        const int c = idx / (BM / 8);
-        const int ch = (idx % (BM / 8)) * 8;
-        *reinterpret_cast<u32x4*>(Xs + c * XLD + ch) = *reinterpret_cast<const u32x4*>(Xb + (size_t)c * pe + ch);
-      }
+    for (int q = 0; q < PL; ++q) *reinterpret_cast<u32x4*>(Xs + poff + q * (NT / (BM / 8)) * XLD) = Xr[q];
+#pragma unroll
+    for (int q = 0; q < XL; ++q) {
+      const int idx = tid + q * NT;
+      float v[XV];
+      unpack16<TZ>(xr[q], v);
+      store_vec<bf16, XV>(A2 + (idx / (C / XV)) * ALD + (idx % (C / XV)) * XV, v);
     }
-    copy_tile_to_lds<TZ, bf16, C, BM, NT>(
-        [&](int p) -> const TZ* { return p < nvalid ? x + (tok0 + p) * C : nullptr; }, A2, ALD);
+    issue_x(next);
     __syncthreads();
 
-    // LN_out statistics (fp32, two-pass) and xln = LN_out(X) into A1 and xln_out
+    // LN_out statistics (fp32, two-pass) and xln = LN_out(X) into A1
+    float mean, rstd;
     {
       float xv[CPQ];
       float sm = 0.f;
 #pragma unroll
       for (int e = 0; e < CPQ; ++e) {
-        xv[e] = to_f32(Xs[(qq * CPQ + e) * XLD + pq]);
+        xv[e] = to_f32(Xs[och(e) * XLD + op]);
         sm += xv[e];
       }
-      const float mean = group_sum<NQ>(sm) * (1.0f / C);
+      mean = dpp_sum8(sm) * (1.0f / C);
       float v = 0.f;
 #pragma unroll
       for (int e = 0; e < CPQ; ++e) {
         const float d = xv[e] - mean;
         v += d * d;
       }
-      const float rstd = rsqrtf(group_sum<NQ>(v) * (1.0f / C) + eps);
-      if (qq == 0) {
-        s_mean[pq] = mean;
-        s_rstd[pq] = rstd;
-      }
-      float y[CPQ];
+      rstd = rsqrtf(dpp_sum8(v) * (1.0f / C) + eps);
 #pragma unroll
-      for (int e = 0; e < CPQ; ++e) y[e] = (xv[e] - mean) * rstd * s_lnw[qq * CPQ + e] + s_lnb[qq * CPQ + e];
-#pragma unroll
-      for (int e = 0; e < CPQ; e += 8) {
-        store_vec<bf16, 8>(A1 + pq * ALD + qq * CPQ + e, y + e);
-        if (pq < nvalid) store_vec<bf16, 8>(xln_out + (tok0 + pq) * C + qq * CPQ + e, y + e);
+      for (int e = 0; e < CPQ; e += 2) {
+        const int c = och(e);
+        const float y[2] = {(xv[e] - mean) * rstd * s_lnw[c] + s_lnb[c],
+                            (xv[e + 1] - mean) * rstd * s_lnw[c + 1] + s_lnb[c + 1]};
+        store_vec<bf16, 2>(A1 + op * ALD + c, y);
       }
     }
     __syncthreads();
@@ -473,43 +503,47 @@ __global__ __launch_bounds__(OutputVjpWs::NT) void trimul_output_vjp_ws_kernel(
     f32x4 accp[4] = {}, accg[4] = {};
     gemm_a_lds_w_regs(accp, A1, ALD, wo);
     gemm_a_lds_w_regs(accg, A2, ALD, wog);
+    // rows of A1 / A2, token-major, for the weight-gradient GEMMs
+    auto rows_out = [&](bf16* dst, const bf16* src) __attribute__((always_inline)) {
+      const auto r = buf_rsrc(dst + t.tok0 * C, row_bytes);
+#pragma unroll
+      for (int q = 0; q < BM * C / 8 / NT; ++q) {
+        const int idx = tid + q * NT;
+        buf_store16(r, *reinterpret_cast<const u32x4*>(src + (idx / (C / 8)) * ALD + (idx % (C / 8)) * 8),
+                    16 * idx);
+      }
+    };
+    rows_out(xln_out, A1);
     __syncthreads();  // A1 / A2 are rewritten below
 
-    // gp = g s, gg = g p s (1 - s), rounded to bf16 as the next GEMMs' operands
+    // gp = g s, gg = g p s (1 - s), rounded to bf16 as the next GEMMs' operands (g is 0 past
+    // the tile's tokens)
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int p = 16 * rb + 4 * (l >> 4) + e;
-        const float gv = p < nvalid ? to_f32(g[(tok0 + p) * C + col]) : 0.f;
+        const float gv = bits_to_f32<TZ>(gr[4 * rb + e]);
         const float sv = sigmoidf_(accg[rb][e]);
         A1[p * ALD + col] = from_f32<bf16>(gv * sv);
         A2[p * ALD + col] = from_f32<bf16>(gv * accp[rb][e] * sv * (1.f - sv));
       }
+    issue_g(next);
     __syncthreads();
-    // gp, gg token-major for the weight-gradient GEMMs
-#pragma unroll
-    for (int it = 0; it < BM * C / 8 / NT; ++it) {
-      const int idx = tid + it * NT;
-      const int p = idx / (C / 8);
-      const int ch = (idx % (C / 8)) * 8;
-      if (p < nvalid) {
-        *reinterpret_cast<u32x4*>(gp_out + (tok0 + p) * C + ch) = *reinterpret_cast<const u32x4*>(A1 + p * ALD + ch);
-        *reinterpret_cast<u32x4*>(gg_out + (tok0 + p) * C + ch) = *reinterpret_cast<const u32x4*>(A2 + p * ALD + ch);
-      }
-    }
 
     // d(xln) = gp Wo, the output gate's x cotangent gg Wog
     f32x4 accd[4] = {}, accx[4] = {};
     gemm_a_lds_w_regs(accd, A1, ALD, wot);
     gemm_a_lds_w_regs(accx, A2, ALD, wogt);
+    rows_out(gp_out, A1);
+    rows_out(gg_out, A2);
+    {
+      const auto r = buf_rsrc(gx + t.tok0 * C, 2 * row_bytes);
+      const int off = (4 * (l >> 4) * C + col) * 4;
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int p = 16 * rb + 4 * (l >> 4) + e;
-        if (p < nvalid) gx[(tok0 + p) * C + col] = accx[rb][e];
-      }
+      for (int q = 0; q < 16; ++q)
+        buf_store_elem<float>(r, accx[q >> 2][q & 3], off + (16 * (q >> 2) + (q & 3)) * C * 4);
+    }
     __syncthreads();  // A1 / A2 dead: the fp32 stage takes their place
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb)
@@ -517,66 +551,72 @@ __global__ __launch_bounds__(OutputVjpWs::NT) void trimul_output_vjp_ws_kernel(
       for (int e = 0; e < 4; ++e) stage[(16 * rb + 4 * (l >> 4) + e) * SLD + col] = accd[rb][e];
     __syncthreads();
 
-    // LN_out affine partials: channel tid & 127 over positions 16 (tid >> 7) .. +16 (positions
-    // past N have d = 0)
+    // LN_out pullback, in place over Xs (each thread its own entries), and the affine partials
+    // (positions past the tile's tokens have d = 0)
     {
-      const int c = tid & (C - 1);
-      const int p0 = 16 * (tid >> 7);
-#pragma unroll 4
-      for (int p = p0; p < p0 + 16; ++p) {
-        const float xn = (to_f32(Xs[c * XLD + p]) - s_mean[p]) * s_rstd[p];
-        const float d = stage[p * SLD + c];
-        pw += d * xn;
-        pb += d;
-      }
-    }
-    __syncthreads();  // Xs is overwritten with dX below
-
-    // LN_out pullback, in place over Xs: each thread owns (position pq, channels qq*CPQ..)
-    {
-      const float mean = s_mean[pq], rstd = s_rstd[pq];
       float u[CPQ], xn[CPQ];
       float su = 0.f, sux = 0.f;
 #pragma unroll
       for (int e = 0; e < CPQ; ++e) {
-        const int c = qq * CPQ + e;
-        xn[e] = (to_f32(Xs[c * XLD + pq]) - mean) * rstd;
-        u[e] = stage[pq * SLD + c] * s_lnw[c];
+        const int c = och(e);
+        xn[e] = (to_f32(Xs[c * XLD + op]) - mean) * rstd;
+        const float d = stage[op * SLD + c];
+        pw[e] += d * xn[e];
+        pb[e] += d;
+        u[e] = d * s_lnw[c];
         su += u[e];
         sux += u[e] * xn[e];
       }
-      su = group_sum<NQ>(su) * (1.0f / C);
-      sux = group_sum<NQ>(sux) * (1.0f / C);
+      su = dpp_sum8(su) * (1.0f / C);
+      sux = dpp_sum8(sux) * (1.0f / C);
 #pragma unroll
-      for (int e = 0; e < CPQ; ++e)
-        Xs[(qq * CPQ + e) * XLD + pq] = from_f32<bf16>(rstd * (u[e] - su - xn[e] * sux));
+      for (int e = 0; e < CPQ; ++e) Xs[och(e) * XLD + op] = from_f32<bf16>(rstd * (u[e] - su - xn[e] * sux));
     }
     __syncthreads();
     {
-      bf16* Db = dX + (size_t)b * C * pe + (size_t)i * Np + j0;
+      bf16* Db = dX + (size_t)t.b * C * pe + (size_t)t.i * Np + t.j0 + (size_t)(tid / (BM / 8)) * pe +
+                 8 * (tid % (BM / 8));
 #pragma unroll
-      for (int it = 0; it < C * BM / 8 / NT; ++it) {
-        const int idx = tid + it * NT;
-        const int c = idx / (BM / 8);
-        const int ch = (idx % (BM / 8)) * 8;
-        *reinterpret_cast<u32x4*>(Db + (size_t)c * pe + ch) = *reinterpret_cast<const u32x4*>(Xs + c * XLD + ch);
-      }
+      for (int q = 0; q < PL; ++q)
+        *reinterpret_cast<u32x4*>(Db + (size_t)q * (NT / (BM / 8)) * pe) =
+            *reinterpret_cast<const u32x4*>(Xs + poff + q * (NT / (BM / 8)) * XLD);
     }
     __syncthreads();  // Xs, A1 / A2 and the stage free for the next tile
   }
-  // this block's partials: the four position quarters added in order
-  red[0][tid] = pw;
-  red[1][tid] = pb;
-  __syncthreads();
-  if (tid < C) {
-    float sw = 0.f, sb = 0.f;
+  // tiles of padding only: dX is zero there (the contraction's cotangent GEMMs read it)
+  {
+    const int tpp = Np / BM;
+    for (int pt = blockIdx.x; pt < B * Np * tpp; pt += G) {
+      const int row = pt / tpp;  // b Np + i
+      const int j0 = (pt - row * tpp) * BM;
+      if (row % Np < N && j0 < N) continue;
+      bf16* Db = dX + (size_t)(row / Np) * C * pe + (size_t)(row % Np) * Np + j0 + (size_t)(tid / (BM / 8)) * pe +
+                 8 * (tid % (BM / 8));
 #pragma unroll
-    for (int q = 0; q < NT / C; ++q) {
-      sw += red[0][q * C + tid];
-      sb += red[1][q * C + tid];
+      for (int q = 0; q < PL; ++q)
+        *reinterpret_cast<u32x4*>(Db + (size_t)q * (NT / (BM / 8)) * pe) = u32x4{0u, 0u, 0u, 0u};
     }
-    partial[(size_t)blockIdx.x * 2 * C + tid] = sw;
-    partial[(size_t)blockIdx.x * 2 * C + C + tid] = sb;
+  }
+  // this block's partials: positions of a wave by lane exchanges, then the eight waves in order
+  float* red = stage;  // [wave][2][C]
+#pragma unroll
+  for (int e = 0; e < CPQ; ++e) {
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1) {
+      pw[e] += __shfl_xor(pw[e], o, 64);
+      pb[e] += __shfl_xor(pb[e], o, 64);
+    }
+    if (l < 8) {
+      red[(2 * w) * C + och(e)] = pw[e];
+      red[(2 * w + 1) * C + och(e)] = pb[e];
+    }
+  }
+  __syncthreads();
+  if (tid < 2 * C) {
+    float sum = 0.f;
+#pragma unroll
+    for (int q = 0; q < NT / 64; ++q) sum += red[2 * q * C + tid];
+    partial[(size_t)blockIdx.x * 2 * C + tid] = sum;
   }
 }
 
@@ -813,7 +853,11 @@ __global__ __launch_bounds__(vjp_nt<C>()) void trimul_project_vjp_kernel(const T
 // at a time (registers for all sixteen would cost the occupancy). Per tile: x rows -> LDS (bf16), each
 // wave's cotangent rows (32 channels x 64 positions of dP or dQ) -> its private LDS stage,
 // both loaded a tile ahead into registers; acc^T, G in registers, G rows -> the LDS G tile;
-// then G leaves token-major (1 KB rows) and dx = gx_in + G W4 is formed from the G tile.
+// then dx = gx_in + G W4 is formed from the G tile and G leaves token-major (1 KB rows). All
+// token accesses are buffer accesses without branches, gx is loaded before the product and
+// nothing is loaded behind the tile's 72 KB of stores: with gx loaded element by element behind
+// its bounds test after them, a tile was sixteen round trips (171 us at B = 1, N = 384, now
+// 103; its bytes take 73).
 struct ProjectVjpWs {
   static constexpr int C = 128;
   static constexpr int BP = 64;         // positions per tile
@@ -885,7 +929,8 @@ __global__ __launch_bounds__(ProjectVjpWs::NT) void trimul_project_vjp_ws_kernel
       const int ch = (idx % (C / XV)) * XV;
       xr[q] = *reinterpret_cast<const u32x4*>(x + tok(b, line, min(t0 + p, N - 1)) * C + ch);
     }
-    if (tid < BP) mr = t0 + tid < N ? mask[tok(b, line, t0 + tid)] : 0.f;
+    mr = mask[tok(b, line, min(t0 + (tid & (BP - 1)), N - 1))];
+    mr = t0 + (tid & (BP - 1)) < N ? mr : 0.f;
     const bf16* cb = dplanes + ((size_t)(pl * B + b) * C + 32 * cj) * pe + (size_t)line * Np + t0 + 8 * (l & 7);
 #pragma unroll
     for (int it = 0; it < 4; ++it) cr[it] = *reinterpret_cast<const u32x4*>(cb + (size_t)(8 * it + (l >> 3)) * pe);
@@ -912,7 +957,7 @@ __global__ __launch_bounds__(ProjectVjpWs::NT) void trimul_project_vjp_ws_kernel
     int b, line, t0;
     tile_coords(tile, b, line, t0);
     stage();
-    if (tile + G < ntiles) issue(tile + G);
+    issue(min(tile + G, ntiles - 1));
     __syncthreads();  // x tile, masks and stages of this tile
 
     // acc^T [row][position] per 32-position half, then G = (g s, g p s (1 - s)) into gs.
@@ -946,32 +991,23 @@ __global__ __launch_bounds__(ProjectVjpWs::NT) void trimul_project_vjp_ws_kernel
     }
     __syncthreads();  // G tile
 
-    // G rows token-major (walk order), 1 KB each; x rows in walk order for the incoming
-    // direction.
     const int nvalid = min(BP, N - t0);
-    bf16* gdst = gpg + (((size_t)b * N + line) * N + t0) * 4 * C;
-#pragma unroll
-    for (int it = 0; it < BP * 4 * C / 8 / NT; ++it) {
-      const int idx = tid + it * NT;
-      const int p = idx / (4 * C / 8);
-      const int ch = (idx % (4 * C / 8)) * 8;
-      if (p < nvalid)
-        *reinterpret_cast<u32x4*>(gdst + (size_t)p * 4 * C + ch) = *reinterpret_cast<const u32x4*>(gs + p * GLD + ch);
-    }
-    if (!outgoing) {
-      bf16* xdst = xw + (((size_t)b * N + line) * N + t0) * C;
-#pragma unroll
-      for (int it = 0; it < BP * C / 8 / NT; ++it) {
-        const int idx = tid + it * NT;
-        const int p = idx / (C / 8);
-        const int ch = (idx % (C / 8)) * 8;
-        if (p < nvalid)
-          *reinterpret_cast<u32x4*>(xdst + (size_t)p * C + ch) = *reinterpret_cast<const u32x4*>(xs + p * XLD + ch);
-      }
-    }
-
-    // dx [position][16 w + (l & 15)] = gx_in + G W4 (k = 4C in 32-row steps)
+    // Position p of the tile is token tbase + p tstr; buffer accesses, zero or dropped past the
+    // tile's tokens. gx is asked for before the product that it is added to, and the stores
+    // come last: a load behind them would wait for them.
+    const long tbase = tok(b, line, t0);
+    const int tstr = outgoing ? 1 : N;
     const int c = 16 * w + (l & 15);
+    const unsigned rows = (unsigned)(nvalid - 1) * tstr * C + C;  // elements up to the last token's end
+    float gxv[BP / 4];
+    {
+      const auto rg = buf_rsrc(gx_in + tbase * C, rows * 4);
+      const int off = (4 * (l >> 4) * tstr * C + c) * 4;
+#pragma unroll
+      for (int q = 0; q < BP / 4; ++q)
+        gxv[q] = __uint_as_float(buf_load_bits<float>(rg, off + (16 * (q >> 2) + (q & 3)) * tstr * C * 4));
+    }
+    // dx [position][16 w + (l & 15)] = gx_in + G W4 (k = 4C in 32-row steps)
     f32x4 acc2[BP / 16] = {};
 #pragma unroll 1
     for (int s4 = 0; s4 < 4 * C / 32; s4 += 4) {
@@ -987,18 +1023,35 @@ __global__ __launch_bounds__(ProjectVjpWs::NT) void trimul_project_vjp_ws_kernel
           acc2[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gf, wb[u], acc2[rb], 0, 0, 0);
         }
     }
-    // position p of the tile is token tbase + p tstr
-    const long tbase = tok(b, line, t0);
-    const long tstr = outgoing ? 1 : N;
-    const float* gxt = gx_in + tbase * C + c;
-    TZ* dxt = dx + tbase * C + c;
+    {
+      const auto rd = buf_rsrc(dx + tbase * C, rows * (int)sizeof(TZ));
+      const int off = (4 * (l >> 4) * tstr * C + c) * (int)sizeof(TZ);
 #pragma unroll
-    for (int rb = 0; rb < BP / 16; ++rb)
+      for (int q = 0; q < BP / 4; ++q)
+        buf_store_elem<TZ>(rd, gxv[q] + acc2[q >> 2][q & 3],
+                           off + (16 * (q >> 2) + (q & 3)) * tstr * C * (int)sizeof(TZ));
+    }
+    // G rows token-major (walk order), 1 KB each; x rows in walk order for the incoming
+    // direction.
+    const long walk = ((long)b * N + line) * N + t0;
+    {
+      const auto rg = buf_rsrc(gpg + walk * 4 * C, nvalid * 4 * C * 2);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int p = 16 * rb + 4 * (l >> 4) + r;
-        if (p < nvalid) dxt[p * tstr * C] = from_f32<TZ>(gxt[p * tstr * C] + acc2[rb][r]);
+      for (int it = 0; it < BP * 4 * C / 8 / NT; ++it) {
+        const int idx = tid + it * NT;
+        buf_store16(rg, *reinterpret_cast<const u32x4*>(gs + (idx / (4 * C / 8)) * GLD + (idx % (4 * C / 8)) * 8),
+                    16 * idx);
       }
+    }
+    if (!outgoing) {
+      const auto rx = buf_rsrc(xw + walk * C, nvalid * C * 2);
+#pragma unroll
+      for (int it = 0; it < BP * C / 8 / NT; ++it) {
+        const int idx = tid + it * NT;
+        buf_store16(rx, *reinterpret_cast<const u32x4*>(xs + (idx / (C / 8)) * XLD + (idx % (C / 8)) * 8),
+                    16 * idx);
+      }
+    }
     __syncthreads();  // x tile, stages and G tile free for the next tile
   }
 }

@@ -150,3 +150,34 @@ def test_trimul_backward_is_deterministic(dev):
         grads.append([x.grad.clone()] + [p.grad.clone() for p in m.parameters()])
     for a, b in zip(*grads):
         assert torch.equal(a, b)
+
+
+# 1: one token; 65: a whole tile and one token of the next; 129: a ragged tile and 127 rows and
+# columns of padding planes; more tiles than one per CU, and B > 1
+@pytest.mark.parametrize("outgoing", [True, False], ids=["out", "in"])
+@pytest.mark.parametrize("xdtype", [torch.float32, BF], ids=["x32", "x16"])
+@pytest.mark.parametrize("B,N", [(1, 1), (2, 65), (1, 129)])
+def test_persistent_vjps_against_fp64(dev, B, N, xdtype, outgoing):
+    """bf16 GEMM operands at C = 128 (the persistent VJP kernels): every gradient within four
+    roundings to bf16 (2^-8 relL2 each: x or G, the planes, their cotangents, the result) of the
+    fp64 gradients on the same bf16 operands."""
+    C = 128
+    x, mask, ws, cot = _core_inputs(B, N, C, seed=900 + N)
+    if N < 3:
+        mask.fill_(1.0)
+    x, cot = x.to(xdtype), cot.to(xdtype)
+    print(f"[trimul vjp bf16] B={B} N={N} x {xdtype} outgoing={outgoing}", flush=True)
+    leaves = [x.to(dev).requires_grad_(True)] + [t.to(dev).requires_grad_(True) for t in ws]
+    with torch.autocast("cuda", dtype=BF):
+        out = kernels.FusedTriMulFunction.apply(leaves[0], mask.to(dev), *leaves[1:], 1e-5, outgoing)
+    got = torch.autograd.grad(out, leaves, grad_outputs=cot.to(dev))
+    r = lambda t: t.to(BF).double()  # noqa: E731
+    ref_in = [r(x), r(ws[0]), r(ws[1]), ws[2].double(), ws[3].double(), r(ws[4]), r(ws[5])]
+    ref_leaves = [t.requires_grad_(True) for t in ref_in]
+    ref = R.tri_mul_core(ref_leaves[0], mask.double(), *ref_leaves[1:], 1e-5, outgoing)
+    want = torch.autograd.grad(ref, ref_leaves, grad_outputs=cot.double())
+    for a, b, name in zip((out.detach(),) + got, (ref.detach(),) + want, ("update",) + NAMES):
+        assert a.shape == b.shape and torch.isfinite(a).all(), name
+        e = rel_l2(a.double().cpu(), b)
+        print(f"  {name}: relL2 {e:.2e}", flush=True)
+        assert e <= 4 * 2.0**-8, name
