@@ -1191,6 +1191,8 @@ __global__ __launch_bounds__(ProjectWs::NT) void trimul_project_ws_kernel(
 // residual; after the MFMAs each wave stages its fp32 update block-wide, and each wave then
 // adds the update to the 8 z rows it loaded and writes them. The next tile's X and z are
 // loaded during this tile's MFMAs.
+// LN_IN = false takes z as given: the training forward's K3, whose x is normalised already
+// (50 -> 30 us against the tile kernel at N = 384).
 struct OutputWs {
   static constexpr int C = 128;
   static constexpr int BP = 64;
@@ -1201,7 +1203,7 @@ struct OutputWs {
   static constexpr int SLD = C + 4;   // fp32 update stage rows [pos][ch]
 };
 
-template <class TZ>
+template <class TZ, bool LN_IN>
 __global__ __launch_bounds__(OutputWs::NT) void trimul_output_ws_kernel(
     const bf16* __restrict__ X, const TZ* __restrict__ z, TZ* __restrict__ out, const float* __restrict__ lniw,
     const float* __restrict__ lnib, float eps_in, const float* __restrict__ lnow, const float* __restrict__ lnob,
@@ -1240,8 +1242,8 @@ __global__ __launch_bounds__(OutputWs::NT) void trimul_output_ws_kernel(
   float liw[VEC], lib[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; ++e) {
-    liw[e] = lniw[chunk * VEC + e];
-    lib[e] = lnib[chunk * VEC + e];
+    liw[e] = LN_IN ? lniw[chunk * VEC + e] : 1.f;
+    lib[e] = LN_IN ? lnib[chunk * VEC + e] : 0.f;
   }
   // LN_out: thread (position op = tid / 8, part os = tid % 8) normalises the channel pairs
   // 16 k + 2 os + {0, 1}, k = 0..7: the 64 lanes of one read instruction touch 32 distinct
@@ -1297,20 +1299,25 @@ __global__ __launch_bounds__(OutputWs::NT) void trimul_output_ws_kernel(
 #pragma unroll
     for (int q = 0; q < NLD; ++q) {
       unpack16<TZ>(zr[q], zv[q]);
-      float sum = 0.f;
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) sum += zv[q][e];
-      const float mean = row_group_sum<LPR>(sum) * (1.0f / C);
-      float sq = 0.f;
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        const float d = zv[q][e] - mean;
-        sq += d * d;
-      }
-      const float rstd = rsqrtf(row_group_sum<LPR>(sq) * (1.0f / C) + eps_in);
       float y[VEC];
+      if constexpr (LN_IN) {
+        float sum = 0.f;
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) y[e] = (zv[q][e] - mean) * rstd * liw[e] + lib[e];
+        for (int e = 0; e < VEC; ++e) sum += zv[q][e];
+        const float mean = row_group_sum<LPR>(sum) * (1.0f / C);
+        float sq = 0.f;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          const float d = zv[q][e] - mean;
+          sq += d * d;
+        }
+        const float rstd = rsqrtf(row_group_sum<LPR>(sq) * (1.0f / C) + eps_in);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) y[e] = (zv[q][e] - mean) * rstd * liw[e] + lib[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) y[e] = zv[q][e];
+      }
       store_vec<bf16, VEC>(xb + (w * RPW + q * RPI + l / LPR) * XLD + chunk * VEC, y);
     }
     const int next = tile + gridDim.x;
@@ -1779,9 +1786,8 @@ __global__ void trimul_pack_kernel(const TS* __restrict__ wp, const TS* __restri
   }
 }
 
-// C = 128 in bf16 runs the persistent weight-stationary K1/K3 and C = 256 with bf16 z the
-// persistent weight-streaming K1 and weight-stationary K3 (bf16 GEMMs, either stream); fp32
-// GEMMs and 64 channels (the template stack) run the generic tile kernels.
+// C = 128 in bf16 runs the persistent weight-stationary K1/K3 and C = 256 the persistent
+// weight-streaming K1 and weight-stationary K3 (bf16 GEMMs, either stream); fp32 GEMMs and 64 channels (the template stack) run the generic tile kernels.
 // mx.heads > 0 runs the MHR mix in K3 (always the generic K3).
 template <class TZ, class TC, int C>
 int trimul_launch(const void* z, const float* mask, const float* lniw, const float* lnib, float eps_in,
@@ -1861,9 +1867,10 @@ int trimul_launch(const void* z, const float* mask, const float* lniw, const flo
       PF_REQUIRE(ntiles < (1L << 31) && (long)Np * Np * OutputWs::C < (1L << 31), PF_ERR_UNSUPPORTED,
                  "trimul_output: N=%d B=%d (B N ceil(N/64) and 128 Np^2 must stay below 2^31)", N, B);
       const int nblk = (int)std::min<long>(ntiles, pf::cu_count());
-      trimul_output_ws_kernel<TZ><<<nblk, OutputWs::NT, 0, s>>>((const bf16*)X, (const TZ*)z, (TZ*)out, lniw, lnib,
-                                                                eps_in, lnow, lnob, eps_out, (const bf16*)wo,
-                                                                (const bf16*)wog, B, N, Np, accumulate);
+      trimul_output_ws_kernel<TZ, true><<<nblk, OutputWs::NT, 0, s>>>((const bf16*)X, (const TZ*)z, (TZ*)out, lniw,
+                                                                      lnib, eps_in, lnow, lnob, eps_out,
+                                                                      (const bf16*)wo, (const bf16*)wog, B, N, Np,
+                                                                      accumulate);
       (void)grid;
     } else if constexpr (sizeof(TC) == 2 && C == 256) {
       const long ntiles = (long)B * N * ((N + Output256::BP - 1) / Output256::BP);
@@ -1937,6 +1944,17 @@ int trimul_train_launch(const void* x, const float* mask, const void* w4, const 
     e = contract_generic_launch<TC>(P, Q, X, G, Np, remap, s);
   }
   if (e) return e;
+  if constexpr (sizeof(TC) == 2 && C == 128) {
+    // the persistent K3 without its LayerNorm of z, within its 32-bit offsets
+    const long ntiles = (long)B * N * ((N + OutputWs::BP - 1) / OutputWs::BP);
+    if (mx.heads == 0 && ntiles < (1L << 31) && (long)pe * C < (1L << 31)) {
+      const int nblk = (int)std::min<long>(ntiles, pf::cu_count());
+      trimul_output_ws_kernel<TZ, false><<<nblk, OutputWs::NT, 0, s>>>((const bf16*)X, (const TZ*)x, (TZ*)out, nullptr,
+                                                                       nullptr, 0.f, lnow, lnob, eps_out,
+                                                                       (const bf16*)wo, (const bf16*)wog, B, N, Np, 0);
+      return pf::check_launch("trimul_train_output");
+    }
+  }
   if (mx.heads > kMhrHeadsSmall)
     trimul_output_kernel<TZ, TC, C, false, true><<<dim3((N + BM - 1) / BM, N, B), trimul_nt<C>(), 0, s>>>(
         X, (const TZ*)x, (TZ*)out, nullptr, nullptr, 0.f, lnow, lnob, eps_out, (const TC*)wo, (const TC*)wog, B, N,
