@@ -448,11 +448,24 @@ def _split_chunk(M: int, target: int = 4096) -> int:
 
 def _weight_grad_tm(gy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """``gy^T x`` (fp32, or fp64 for fp64 operands) for token-major gy [M, Co] and x [M, Ci]
-    with M in the hundreds of thousands: the tokens split into chunks of a batched GEMM (one
-    [Co, Ci] tile alone leaves the GPU idle; left operand a strided view, right operand
-    contiguous), summed over chunks."""
+    with M in the hundreds of thousands: bf16 operands in multiples of 128 channels on
+    ``pf_weight_grad`` (512 x 128 over 384^2 tokens: 38 us against 70); others as a batched
+    GEMM over chunks of tokens (one [Co, Ci] tile alone leaves the GPU idle; left operand a
+    strided view, right operand contiguous), summed over chunks."""
     acc = torch.promote_types(gy.dtype, torch.float32)
-    M = gy.shape[0]
+    M, Co = gy.shape
+    Ci = x.shape[1]
+    if gy.dtype == x.dtype == torch.bfloat16 and gy.is_cuda and Co % 128 == 0 and Ci % 128 == 0:
+        gy, x = gy.contiguous(), x.contiguous()
+        ws_bytes = _lib.lib().pf_weight_grad_workspace_bytes(M, Co, Ci)
+        if (gy.data_ptr() | x.data_ptr()) % 16 == 0 and M < 2**31 - 65536 and Co * Ci < 2**30:
+            out = torch.empty((Co, Ci), dtype=torch.float32, device=gy.device)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=gy.device)
+            _lib.call(
+                "pf_weight_grad", gy.data_ptr(), x.data_ptr(), M, Co, Ci, _lib.PF_BF16, out.data_ptr(), ws.data_ptr(),
+                ws_bytes, _lib.stream_of(gy),
+            )  # fmt: skip
+            return out
     chunk = _split_chunk(M)
     S = M // chunk
     m0 = S * chunk

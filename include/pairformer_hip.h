@@ -447,6 +447,12 @@ size_t pf_layernorm_linear_workspace_bytes(long M, int K, int cdtype);
 int pf_layernorm_linear_fwd(const void* x, int xdtype, const float* ln_w, const float* ln_b, float eps,
                             const void* w_nk, const float* bias, long M, int K, int Nout, int cdtype, void* out,
                             void* workspace, size_t workspace_bytes, void* stream);
+/* Weight gradient of a linear (the weight's VJP of F.linear): out [Co, Ci] fp32 = gy^T x for
+ * token-major gy [M, Co] and x [M, Ci] in bf16, Co and Ci multiples of 128; fp32 sums in a
+ * fixed order. Pointers 16-byte aligned. */
+size_t pf_weight_grad_workspace_bytes(long M, int Co, int Ci);
+int pf_weight_grad(const void* gy, const void* x, long M, int Co, int Ci, int dtype, float* out, void* workspace,
+                   size_t workspace_bytes, void* stream);
 /* FusedSwiGLU()(x) (triton/swiglu.py:192-200): y [M, D] = silu(x[:, :D]) * x[:, D:], x [M, 2D]. */
 int pf_swiglu_fwd(const void* x, int dtype, void* y, long M, int D, void* stream);
 /* Backward of pf_swiglu_fwd (FusedSwiGLU's VJP, triton/swiglu.py:60-95): dx [M, 2D] from

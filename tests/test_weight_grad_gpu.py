@@ -1,0 +1,44 @@
+"""Split weight gradient of a linear over token-major bf16 operands (``pf_weight_grad``) on a
+real MI355X, against the fp64 product of the same operands."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tests._helpers import mod
+
+pytestmark = pytest.mark.gpu
+
+kernels = mod("kernels")
+
+
+@pytest.fixture(scope="module")
+def dev():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    return torch.device("cuda:0")
+
+
+# 1: one token, every other chunk empty; 63..65: around the 64-token step; 8191: a ragged last
+# chunk; 40000: the smallest sizes that the training path splits; Co, Ci: one tile, several
+# tiles of either operand, a tile count that does not divide the CUs
+@pytest.mark.parametrize("M,Co,Ci", [
+    (1, 128, 128), (63, 128, 128), (64, 256, 128), (65, 128, 256), (8191, 512, 128), (40000, 128, 512),
+    (40001, 384, 256),
+])  # fmt: skip
+def test_weight_grad_against_fp64(dev, M, Co, Ci):
+    """fp32 products and sums: within 8 roundings of the terms' magnitudes (a chain of M terms
+    split over steps, groups and chunks), bitwise the same on a second run."""
+    g = torch.Generator().manual_seed(M + Co)
+    gy = torch.randn(M, Co, generator=g).to(dev, torch.bfloat16)
+    x = torch.randn(M, Ci, generator=g).to(dev, torch.bfloat16)
+    print(f"[weight grad] M={M} Co={Co} Ci={Ci}", flush=True)
+    out = kernels._weight_grad_tm(gy, x)
+    assert out.dtype == torch.float32 and out.shape == (Co, Ci)
+    want = gy.double().t() @ x.double()
+    mag = gy.double().abs().t() @ x.double().abs()
+    worst = ((out.double() - want).abs() / (mag * 2.0**-23 * 8 + 1e-30)).max().item()
+    print(f"  {worst:.3f} of the bound", flush=True)
+    assert worst <= 1.0
+    assert torch.equal(out, kernels._weight_grad_tm(gy, x))
