@@ -149,64 +149,118 @@ __global__ __launch_bounds__(256) void layernorm128_kernel(const T* __restrict__
 }
 
 // ------------------------------------------------------------------ backward
-// One wave per row, kLnbRows rows per block; each lane owns C / 64 consecutive channels.
-// dx = rstd (g - mean(g) - xn mean(g xn)) with g = dy * w and xn the standardised x
-// (statistics recomputed, fp32 two-pass as the forward); per-block partial sums of
-// dy * xn (weight) and dy (bias), added in block order by ln_param_grad_reduce.
+// 16 lanes per row (32 from 256 channels), kLnbRows rows per block; a lane owns runs of four
+// channels, so its loads and stores are 8 or 16 bytes (VEC: the operands are 16-byte aligned;
+// element accesses otherwise) and a row's four sums stay within its lanes. dx = rstd (g -
+// mean(g) - xn mean(g xn)) with g = dy * w and xn the standardised x (statistics recomputed,
+// fp32 two-pass as the forward); per-block partial sums of dy * xn (weight) and dy (bias),
+// added in block order by ln_param_grad_reduce. Bytes bound it: 147456 x 128 with fp32 x and
+// bf16 dy 33 us (its bytes at the rate of a large copy: 36); with a wave per row, two channels per lane and 64-lane sums it
+// took 55.
 constexpr int kLnbRows = 64;
 
-template <class T, int C, class TD = T>
+template <bool VEC, class T>
+PF_DEVICE f32x4 load4(const T* p) {
+  if constexpr (!VEC) {
+    return f32x4{to_f32(p[0]), to_f32(p[1]), to_f32(p[2]), to_f32(p[3])};
+  } else if constexpr (sizeof(T) == 2) {
+    const bf16x4 v = *reinterpret_cast<const bf16x4*>(p);
+    return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+  } else {
+    return *reinterpret_cast<const f32x4*>(p);
+  }
+}
+
+template <class T, int C, class TD, bool VEC>
 __global__ __launch_bounds__(256) void layernorm_bwd_kernel(const T* __restrict__ x, const TD* __restrict__ dy,
                                                             const float* __restrict__ w, float eps, long M,
                                                             T* __restrict__ dx, float* __restrict__ partial) {
-  constexpr int CPL = C / 64;  // channels per lane
-  __shared__ float red[4][2 * C];
+  constexpr int LPR = C >= 256 ? 32 : 16;  // lanes per row
+  constexpr int STEP = 4 * LPR;            // channels of one run of all lanes
+  constexpr int CH = C / STEP;             // runs per lane
+  constexpr int RPW = 64 / LPR;            // rows per wave and step
+  __shared__ __attribute__((aligned(16))) float red[4][2 * C];
   const int wv = wave_id();
   const int l = lane_id();
-  float wl[CPL], sw[CPL], sb[CPL];
+  const int sub = 4 * (l & (LPR - 1));
+  f32x4 wl[CH], sw[CH], sb[CH];
 #pragma unroll
-  for (int e = 0; e < CPL; ++e) {
-    wl[e] = w[l * CPL + e];
-    sw[e] = sb[e] = 0.f;
+  for (int k = 0; k < CH; ++k) {
+    wl[k] = load4<false>(w + STEP * k + sub);
+    sw[k] = sb[k] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  for (int rr = wv; rr < kLnbRows; rr += 4) {
-    const long r = (long)blockIdx.x * kLnbRows + rr;
-    if (r >= M) break;
-    float xv[CPL], gv[CPL], dv[CPL];
+#pragma unroll 2
+  for (int it = 0; it < kLnbRows / (4 * RPW); ++it) {
+    const long r = (long)blockIdx.x * kLnbRows + (4 * it + wv) * RPW + l / LPR;
+    const long rc = min(r, M - 1);  // rows past the last read it and contribute nothing
+    f32x4 xv[CH], dv[CH];
     float s = 0.f;
 #pragma unroll
-    for (int e = 0; e < CPL; ++e) {
-      xv[e] = to_f32(x[r * C + l * CPL + e]);
-      dv[e] = to_f32(dy[r * C + l * CPL + e]);
-      s += xv[e];
+    for (int k = 0; k < CH; ++k) {
+      xv[k] = load4<VEC>(x + rc * C + STEP * k + sub);
+      dv[k] = load4<VEC>(dy + rc * C + STEP * k + sub);
     }
-    const float mean = group_sum<64>(s) * (1.0f / C);
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+      s += (xv[k][0] + xv[k][1]) + (xv[k][2] + xv[k][3]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dv[k][e] = r < M ? dv[k][e] : 0.f;
+    }
+    const float mean = row_group_sum<LPR>(s) * (1.0f / C);
     float q = 0.f;
 #pragma unroll
-    for (int e = 0; e < CPL; ++e) {
-      const float d = xv[e] - mean;
-      q += d * d;
-    }
-    const float rstd = rsqrtf(group_sum<64>(q) * (1.0f / C) + eps);
+    for (int k = 0; k < CH; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        xv[k][e] -= mean;
+        q += xv[k][e] * xv[k][e];
+      }
+    const float rstd = rsqrtf(row_group_sum<LPR>(q) * (1.0f / C) + eps);
     float sg = 0.f, sgx = 0.f;
 #pragma unroll
-    for (int e = 0; e < CPL; ++e) {
-      xv[e] = (xv[e] - mean) * rstd;  // xn
-      gv[e] = dv[e] * wl[e];
-      sg += gv[e];
-      sgx += gv[e] * xv[e];
-      sw[e] += dv[e] * xv[e];
-      sb[e] += dv[e];
-    }
-    sg = group_sum<64>(sg) * (1.0f / C);
-    sgx = group_sum<64>(sgx) * (1.0f / C);
+    for (int k = 0; k < CH; ++k)
 #pragma unroll
-    for (int e = 0; e < CPL; ++e) dx[r * C + l * CPL + e] = from_f32<T>(rstd * (gv[e] - sg - xv[e] * sgx));
+      for (int e = 0; e < 4; ++e) {
+        xv[k][e] *= rstd;  // xn
+        sw[k][e] += dv[k][e] * xv[k][e];
+        sb[k][e] += dv[k][e];
+        dv[k][e] *= wl[k][e];  // g
+        sg += dv[k][e];
+        sgx += dv[k][e] * xv[k][e];
+      }
+    sg = row_group_sum<LPR>(sg) * (1.0f / C);
+    sgx = row_group_sum<LPR>(sgx) * (1.0f / C);
+    if (r < M) {
+#pragma unroll
+      for (int k = 0; k < CH; ++k) {
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = rstd * (dv[k][e] - sg - xv[k][e] * sgx);
+        if constexpr (VEC) {
+          store_vec<T, 4>(dx + r * C + STEP * k + sub, y);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) dx[r * C + STEP * k + sub + e] = from_f32<T>(y[e]);
+        }
+      }
+    }
   }
 #pragma unroll
-  for (int e = 0; e < CPL; ++e) {
-    red[wv][l * CPL + e] = sw[e];
-    red[wv][C + l * CPL + e] = sb[e];
+  for (int k = 0; k < CH; ++k)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+#pragma unroll
+      for (int o = LPR; o < 64; o <<= 1) {
+        sw[k][e] += __shfl_xor(sw[k][e], o, 64);
+        sb[k][e] += __shfl_xor(sb[k][e], o, 64);
+      }
+    }
+  if (l < LPR) {
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+      *reinterpret_cast<f32x4*>(&red[wv][STEP * k + sub]) = sw[k];
+      *reinterpret_cast<f32x4*>(&red[wv][C + STEP * k + sub]) = sb[k];
+    }
   }
   __syncthreads();
   for (int k = threadIdx.x; k < 2 * C; k += 256)
@@ -240,10 +294,15 @@ int ln_bwd_launch(const void* x, const void* dy, const float* w, float eps, long
                   float* db, void* ws, hipStream_t s) {
   const long nblk = (M + kLnbRows - 1) / kLnbRows;
   float* partial = static_cast<float*>(ws);
+  const bool vec = pf::aligned16(x) && pf::aligned16(dy) && pf::aligned16(dx);
   auto run = [&](auto cc) {
     constexpr int CC = decltype(cc)::value;
-    layernorm_bwd_kernel<T, CC, TD><<<(unsigned)nblk, 256, 0, s>>>((const T*)x, (const TD*)dy, w, eps, M, (T*)dx,
-                                                                    partial);
+    if (vec)
+      layernorm_bwd_kernel<T, CC, TD, true><<<(unsigned)nblk, 256, 0, s>>>((const T*)x, (const TD*)dy, w, eps, M,
+                                                                           (T*)dx, partial);
+    else
+      layernorm_bwd_kernel<T, CC, TD, false><<<(unsigned)nblk, 256, 0, s>>>((const T*)x, (const TD*)dy, w, eps, M,
+                                                                            (T*)dx, partial);
   };
   switch (C) {
     case 64: run(std::integral_constant<int, 64>{}); break;

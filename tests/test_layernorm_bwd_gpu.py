@@ -16,6 +16,7 @@ import torch.nn.functional as F
 from tests._helpers import assert_fp32_close, mod, rel_l2
 
 pytestmark = pytest.mark.gpu
+_lib = mod("_lib")
 kernels = mod("kernels")
 
 
@@ -138,3 +139,45 @@ def test_fused_ops_are_differentiable_fp32(dev):
                      [t.double().requires_grad_(True) for t in (z, lw, lb)], cot.double())  # fmt: skip
     for a, r, name in zip(got, want, ("x", "w", "b")):
         assert_fp32_close(a.cpu(), r.float(), what=f"FusedLayerNormTranspose d{name}")
+
+
+# one row, a row short of and past the rows of a block (64), rows of the last step missing;
+# channel counts of either lane split; operands that are 16-byte aligned and not
+@pytest.mark.parametrize("offset", [0, 1], ids=["aligned", "unaligned"])
+@pytest.mark.parametrize("xdt,ddt", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16),
+                                     (torch.bfloat16, torch.bfloat16)], ids=["f32", "f32-bf16", "bf16"])  # fmt: skip
+@pytest.mark.parametrize("M,C", [(1, 64), (63, 128), (65, 256), (130, 384), (200, 512)])
+def test_layernorm_backward_edges(dev, M, C, xdt, ddt, offset):
+    """dx within its rounding and 16 fp32 roundings of a row's terms, the affine gradients
+    within M fp32 roundings of theirs, of the fp64 gradients on the same operands."""
+    x, w, b, dy = _case(M, C, M + C)
+
+    def place(t, dt):
+        flat = torch.empty(t.numel() + offset, dtype=dt, device=dev)
+        flat[offset:] = t.to(dev, dt).reshape(-1)
+        return flat[offset:].view(t.shape)
+
+    xg, dyg = place(x, xdt), place(dy, ddt)
+    print(f"[layernorm bwd edges] M={M} C={C} {xdt} {ddt} offset={offset}", flush=True)
+    lib = _lib.lib()
+    ws_bytes = lib.pf_layernorm_bwd_workspace_bytes(M, C)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    dx = place(torch.zeros(M, C), xdt)
+    dw, db = torch.empty(C, device=dev), torch.empty(C, device=dev)
+    wg = w.float().to(dev)
+    _lib.call(
+        "pf_layernorm_bwd_mixed", xg.data_ptr(), _lib.dtype_code(xdt), dyg.data_ptr(), _lib.dtype_code(ddt),
+        wg.data_ptr(), 1e-5, dx.data_ptr(), dw.data_ptr(), db.data_ptr(), M, C, ws.data_ptr(), ws_bytes,
+        _lib.stream_of(xg),
+    )  # fmt: skip
+    xd = xg.double().cpu().requires_grad_(True)
+    wd, bd = w.double().requires_grad_(True), b.double().requires_grad_(True)
+    dyd = dyg.double().cpu()
+    torch.nn.functional.layer_norm(xd, (C,), wd, bd, 1e-5).backward(dyd)
+    rnd = 2.0**-8 if xdt == torch.bfloat16 else 2.0**-23
+    rstd = 1 / (xd.detach().var(-1, unbiased=False, keepdim=True) + 1e-5).sqrt()
+    scale = (dyd * wd.detach()).abs().amax(-1, keepdim=True) * rstd  # size of a row's terms
+    assert ((dx.double().cpu() - xd.grad).abs() <= rnd * xd.grad.abs() + 64 * 2.0**-23 * scale).all()
+    xn = ((xd - xd.mean(-1, keepdim=True)) * rstd).detach()
+    for got, want, mag in ((dw, wd.grad, (dyd * xn).abs().sum(0)), (db, bd.grad, dyd.abs().sum(0))):
+        assert ((got.double().cpu() - want).abs() <= (M + 16) * 2.0**-23 * mag).all()
