@@ -795,8 +795,11 @@ __global__ __launch_bounds__(64 * kLinesPerBlock, QS == 1 ? 4 : (QS == 2 ? 4 : 2
   // order, the K/V of block kb): after them it issued one step's K/V/mask loads and one bias
   // stage. Then every wave's stage kb is visible, and stage (kb + 2) % 3 (read at kb - 1) is
   // free for the next fill.
+  // The exact mode counts stage kb + 1's loads only: there the compiler sinks the prologue's K/V
+  // loads behind the first barrier, into the branch that uses them, and a count that includes
+  // them let the first key block read its bias before it had landed.
   auto sync_issue = [&](int kb, int u, Frag16<TC>& kn, Frag16<TC>& vn, float& mn) {
-    constexpr int after = KV_LOADS + DL;
+    constexpr int after = FAST ? KV_LOADS + DL : DL;
     static_assert(after < 16, "vmcnt immediate");
     __builtin_amdgcn_s_waitcnt(after | (7 << 4) | (15 << 8));
     __builtin_amdgcn_s_barrier();
@@ -1587,8 +1590,8 @@ __global__ __launch_bounds__(256) void mask_outer_check_kernel(const float* __re
 //
 // One block packs 64 keys (two key blocks) of one (b, s, h): 16-byte loads and stores
 // throughout, V through LDS into Vt[d][slot] (bf16: the key-block tile). Bytes bound it: at
-// 384 lines x 384 keys x 4 heads in bf16 the three operands take 51 us (their bytes: 44); Q and K in one
-// kernel and V in another, with 2-byte V accesses, took 66 us.
+// 384 lines x 384 keys x 4 heads in bf16 the three operands take 51 us (their bytes: 44);
+// Q and K in one kernel and V in another, with 2-byte V accesses, took 66 us.
 template <class TC>
 __global__ __launch_bounds__(256) void evo_pack_qkv_kernel(const TC* __restrict__ q, const TC* __restrict__ k,
                                                            const TC* __restrict__ v, TC* __restrict__ Qw,

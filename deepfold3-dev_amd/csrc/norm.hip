@@ -155,8 +155,8 @@ __global__ __launch_bounds__(256) void layernorm128_kernel(const T* __restrict__
 // mean(g) - xn mean(g xn)) with g = dy * w and xn the standardised x (statistics recomputed,
 // fp32 two-pass as the forward); per-block partial sums of dy * xn (weight) and dy (bias),
 // added in block order by ln_param_grad_reduce. Bytes bound it: 147456 x 128 with fp32 x and
-// bf16 dy 33 us (its bytes at the rate of a large copy: 36); with a wave per row, two channels per lane and 64-lane sums it
-// took 55.
+// bf16 dy 33 us (its bytes at the rate of a large copy: 36); with a wave per row, two channels
+// per lane and 64-lane sums it took 55.
 constexpr int kLnbRows = 64;
 
 template <bool VEC, class T>

@@ -145,6 +145,22 @@ def test_evo_extreme_pair_bias(dev, dtype):
     assert redo > 0, "the exact pass never ran"
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_evo_exact_pass_repeats(dev, dtype):
+    """The exact pass reads its first bias tile only once it is in LDS: with other kernels'
+    contents in LDS in between, every run gives the same bits, within the policy against fp64."""
+    Q, K, V, rm, _ = _inputs(4, 128, dtype, dev, seed=43)
+    g = torch.Generator().manual_seed(46)
+    pb = ((torch.randint(0, 2, (1, 1, 4, 128, 128), generator=g).float() * 2 - 1) * 1e3).to(dev)
+    fill = torch.full((1024, 1024), 7.0, device=dev, dtype=dtype)
+    outs = []
+    for _ in range(24):
+        fill @ fill
+        outs.append(_run_evo(Q, K, V, rm, pb)[0])
+    _check_evo(outs[0], Q, K, V, rm, pb, f"exact pass repeats {dtype}")
+    assert all(torch.equal(outs[0], o) for o in outs[1:])
+
+
 @pytest.mark.parametrize("sigma", [0.1, 1.0, 10.0, 100.0])
 def test_evo_magnitude_sweep(dev, sigma):
     """sigma sweep on Q/K/V (test_evo_attn_robustness.py:405-445). The reference asserts
