@@ -70,8 +70,10 @@ PF_DEVICE float folded_key_mask(const float* km, int N, int key) {
 // w5 [4C + 16][C] (cdtype): rows q | k | v | g | pb (H rows) | zero padding.
 // Block: BM positions of one line; 4 waves in 2 x 2 (positions x channels), each 32x32
 // MFMA tiles. The four 128-row weight chunks go through one LDS buffer, which doubles as
-// the staging tile for the chunk's output.
-template <class TZ, class TC>
+// the staging tile for the chunk's output. Blocks of padding only write their constants. SPLIT:
+// one block per chunk (blockIdx.z = 4 b + chunk; the chunk-3 block also makes the pair bias
+// and the mask), the same sums in a quarter of the time where whole tiles leave CUs idle.
+template <class TZ, class TC, bool SPLIT>
 __global__ __launch_bounds__(256) void attn_project_kernel(const TZ* __restrict__ z, const float* __restrict__ mask,
                                                            const float* __restrict__ lnw, const float* __restrict__ lnb,
                                                            float eps, const TC* __restrict__ w5, TC* __restrict__ Q,
@@ -92,7 +94,9 @@ __global__ __launch_bounds__(256) void attn_project_kernel(const TZ* __restrict_
 
   const int t0 = blockIdx.x * BM;
   const int line = blockIdx.y;
-  const int b = blockIdx.z;
+  const int b = SPLIT ? blockIdx.z >> 2 : blockIdx.z;
+  const int kind0 = SPLIT ? blockIdx.z & 3 : 0;
+  const int kind1 = SPLIT ? kind0 + 1 : 4;
   const int tid = threadIdx.x;
   const int w = wave_id();
   const int l = lane_id();
@@ -103,8 +107,78 @@ __global__ __launch_bounds__(256) void attn_project_kernel(const TZ* __restrict_
     if (line >= N || t >= N) return -1;
     return transpose ? (long)t * N + line : (long)line * N + t;
   };
+  const bool live = line < N && t0 < N;
+  const size_t lineq = (size_t)b * Np + line;  // [b][line] over the padded frame
+  // Chunk `kind` of the outputs, 16 bytes a thread, from the stage (from(offset)).
+  auto emit = [&](int kind, auto from) {
+    if (kind == 0 || kind == 1) {
+      // Q / K: [b][line][h][t][d]; per head BM x D contiguous.
+      TC* dst = (kind == 0 ? Q : K) + lineq * kHeads * Np * kHeadDim;
+      constexpr int CPP = kHeadDim / VEC;  // chunks per (position, head)
+#pragma unroll
+      for (int it = 0; it < BM * kC / VEC / NT; ++it) {
+        const int idx = tid + it * NT;
+        const int hh = idx / (BM * CPP);
+        const int r = idx % (BM * CPP);
+        const int p = r / CPP;
+        const int d0 = (r % CPP) * VEC;
+        *reinterpret_cast<u32x4*>(dst + ((size_t)hh * Np + t0 + p) * kHeadDim + d0) =
+            from(p * LD + hh * kHeadDim + d0);
+      }
+    } else if (kind == 2) {
+      // Vt: [b][line][h][d][slot]
+      TC* dst = Vt + lineq * kHeads * kHeadDim * Np + t0;
+      constexpr int CPR = BM / VEC;
+#pragma unroll
+      for (int it = 0; it < BM * kC / VEC / NT; ++it) {
+        const int idx = tid + it * NT;
+        const int c = idx / CPR;
+        const int s0 = (idx % CPR) * VEC;
+        *reinterpret_cast<u32x4*>(dst + (size_t)c * Np + s0) = from(c * LD + s0);
+      }
+    } else {
+      // G = sigmoid(g): [b][line][t][C]
+      TC* dst = G + (lineq * Np + t0) * kC;
+      constexpr int CPR = kC / VEC;
+#pragma unroll
+      for (int it = 0; it < BM * kC / VEC / NT; ++it) {
+        const int idx = tid + it * NT;
+        const int p = idx / CPR;
+        const int c0 = (idx % CPR) * VEC;
+        *reinterpret_cast<u32x4*>(dst + (size_t)p * kC + c0) = from(p * LD + c0);
+      }
+    }
+  };
+  // The pair bias (from pbs) and the mask slots of the tile.
+  auto emit_bias = [&]() {
+    const bool line_ok = line < N;
+    for (int idx = tid; idx < kHeads * BM; idx += NT) {
+      const int hh = idx / BM;
+      const int p = idx % BM;
+      const int t = t0 + p;
+      const float v = (line_ok && t < N) ? pbs[p][hh] : 0.f;
+      if (transpose)  // key-major [b][h][key = line][query = t]
+        PB[(((size_t)b * kHeads + hh) * Np + line) * Np + t] = v;
+      else  // query-major [b][h][query = line][slot(key = t)]
+        PB[(((size_t)b * kHeads + hh) * Np + line) * Np + (t & ~31) + key_slot(t & 31)] = v;
+    }
+    if (tid < BM) {
+      const int t = t0 + tid;
+      const float v = t < N ? (mks[tid] - 1.0f) * 1e9f * kLog2e : -INFINITY;
+      MA[lineq * Np + (t & ~31) + key_slot(t & 31)] = v;
+    }
+  };
+  if (!live) {  // padding: q k^T and P V are 0 there; no products, no weights
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    const u32x4 half = __builtin_bit_cast(u32x4, sizeof(TC) == 4 ? f32x4{0.5f, 0.5f, 0.5f, 0.5f} : f32x4{});
+    for (int kind = kind0; kind < kind1; ++kind) emit(kind, [&](int) { return kind == 3 ? half : zero; });
+    if (tid < BM) mks[tid] = 0.f;
+    __syncthreads();
+    if (kind1 == 4) emit_bias();
+    return;
+  }
   Rows128<TC, 128, NT> wpf;
-  wpf.load(w5, kC);
+  wpf.load(w5 + (size_t)kind0 * 128 * kC, kC);
   ln_tile_to_lds<TZ, TC, kC, BM, NT>([&](int p) -> const TZ* {
     const long pos = pos_of(p);
     return pos < 0 ? nullptr : zb + pos * kC;
@@ -113,14 +187,13 @@ __global__ __launch_bounds__(256) void attn_project_kernel(const TZ* __restrict_
     const long pos = pos_of(tid);
     mks[tid] = pos < 0 ? 0.f : mask[(size_t)b * N * N + pos];
   }
-  const size_t lineq = (size_t)b * Np + line;  // [b][line] over the padded frame
 
 #pragma unroll 1
-  for (int kind = 0; kind < 4; ++kind) {
+  for (int kind = kind0; kind < kind1; ++kind) {
     __syncthreads();  // previous chunk's stage fully consumed
     wpf.store(WS, LD);
     __syncthreads();
-    if (kind < 3) wpf.load(w5 + (size_t)(kind + 1) * 128 * kC, kC);
+    if (kind + 1 < kind1) wpf.load(w5 + (size_t)(kind + 1) * 128 * kC, kC);
     if (kind != 2) {
       // position-major output: acc^T = W X^T, lane holds 4 consecutive channels
       f32x16 acc[2][PT];
@@ -166,45 +239,10 @@ __global__ __launch_bounds__(256) void attn_project_kernel(const TZ* __restrict_
           }
     }
     __syncthreads();
-    if (kind == 0 || kind == 1) {
-      // Q / K: [b][line][h][t][d]; per head BM x D contiguous.
-      TC* dst = (kind == 0 ? Q : K) + lineq * kHeads * Np * kHeadDim;
-      constexpr int CPP = kHeadDim / VEC;  // chunks per (position, head)
-#pragma unroll
-      for (int it = 0; it < BM * kC / VEC / NT; ++it) {
-        const int idx = tid + it * NT;
-        const int hh = idx / (BM * CPP);
-        const int r = idx % (BM * CPP);
-        const int p = r / CPP;
-        const int d0 = (r % CPP) * VEC;
-        *reinterpret_cast<u32x4*>(dst + ((size_t)hh * Np + t0 + p) * kHeadDim + d0) =
-            *reinterpret_cast<const u32x4*>(WS + p * LD + hh * kHeadDim + d0);
-      }
-    } else if (kind == 2) {
-      // Vt: [b][line][h][d][slot]
-      TC* dst = Vt + lineq * kHeads * kHeadDim * Np + t0;
-      constexpr int CPR = BM / VEC;
-#pragma unroll
-      for (int it = 0; it < BM * kC / VEC / NT; ++it) {
-        const int idx = tid + it * NT;
-        const int c = idx / CPR;
-        const int s0 = (idx % CPR) * VEC;
-        *reinterpret_cast<u32x4*>(dst + (size_t)c * Np + s0) = *reinterpret_cast<const u32x4*>(WS + c * LD + s0);
-      }
-    } else {
-      // G = sigmoid(g): [b][line][t][C]
-      TC* dst = G + (lineq * Np + t0) * kC;
-      constexpr int CPR = kC / VEC;
-#pragma unroll
-      for (int it = 0; it < BM * kC / VEC / NT; ++it) {
-        const int idx = tid + it * NT;
-        const int p = idx / CPR;
-        const int c0 = (idx % CPR) * VEC;
-        *reinterpret_cast<u32x4*>(dst + (size_t)p * kC + c0) = *reinterpret_cast<const u32x4*>(WS + p * LD + c0);
-      }
-    }
+    emit(kind, [&](int o) { return *reinterpret_cast<const u32x4*>(WS + o); });
   }
 
+  if (SPLIT && kind0 != 3) return;
   // Pair bias: one 16-column block (H real columns) over BM rows, BM/4 rows per wave.
   {
     constexpr int RB = BM / 4 / 16;
@@ -220,22 +258,7 @@ __global__ __launch_bounds__(256) void attn_project_kernel(const TZ* __restrict_
     }
   }
   __syncthreads();
-  const bool line_ok = line < N;
-  for (int idx = tid; idx < kHeads * BM; idx += NT) {
-    const int hh = idx / BM;
-    const int p = idx % BM;
-    const int t = t0 + p;
-    const float v = (line_ok && t < N) ? pbs[p][hh] : 0.f;
-    if (transpose)  // key-major [b][h][key = line][query = t]
-      PB[(((size_t)b * kHeads + hh) * Np + line) * Np + t] = v;
-    else  // query-major [b][h][query = line][slot(key = t)]
-      PB[(((size_t)b * kHeads + hh) * Np + line) * Np + (t & ~31) + key_slot(t & 31)] = v;
-  }
-  if (tid < BM) {
-    const int t = t0 + tid;
-    const float v = t < N ? (mks[tid] - 1.0f) * 1e9f * kLog2e : -INFINITY;
-    MA[lineq * Np + (t & ~31) + key_slot(t & 31)] = v;
-  }
+  emit_bias();
 }
 
 // A1, persistent and weight-stationary (bf16 GEMMs). One 512-thread block per CU walks
@@ -1473,8 +1496,14 @@ int grid_attn_launch(const void* z, const float* mask, const float* lnw, const f
                                                                     Np, transpose, qscale);
       (void)grid;
     } else {
-      attn_project_kernel<TZ, TC><<<grid, 256, 0, s>>>((const TZ*)z, mask, lnw, lnb, eps, (const TC*)w5, Qb, Kb,
-                                                       Vb, Gb, PBb, MAb, N, Np, transpose, qscale);
+      // a block holds a CU: split by chunk while four times the tiles still fit in one round
+      // (N = 64: 38 -> 32 us; split with padding blocks that ran the whole kernel: 43)
+      if (4L * B * N * ((N + BM - 1) / BM) <= pf::cu_count())
+        attn_project_kernel<TZ, TC, true><<<dim3(grid.x, grid.y, 4 * B), 256, 0, s>>>(
+            (const TZ*)z, mask, lnw, lnb, eps, (const TC*)w5, Qb, Kb, Vb, Gb, PBb, MAb, N, Np, transpose, qscale);
+      else
+        attn_project_kernel<TZ, TC, false><<<grid, 256, 0, s>>>((const TZ*)z, mask, lnw, lnb, eps, (const TC*)w5, Qb,
+                                                                Kb, Vb, Gb, PBb, MAb, N, Np, transpose, qscale);
     }
     timer.stop();
     if (int e = pf::check_launch("attn_project")) return e;

@@ -33,14 +33,15 @@ constexpr int trimul_nt() { return C >= 256 ? 512 : 256; }
 // Packed weights w4 [4C][C]: for channel block j (16 channels), rows 64j + 16*kind + r,
 // kind 0 = a projection, 1 = a gate, 2 = b projection, 3 = b gate (channel 16j + r).
 // NORM = false takes z as already normalised (the training entry, whose input LayerNorm
-// runs outside).
-template <class TZ, class TC, int C, bool NORM = true>
+// runs outside). Blocks of padding only skip the products. BM_ positions per block: the
+// results do not depend on it (a position's sums are its own).
+template <class TZ, class TC, int C, bool NORM = true, int BM_ = trimul_bm<TC>()>
 __global__ __launch_bounds__(trimul_nt<C>()) void trimul_project_kernel(const TZ* __restrict__ z, const float* __restrict__ mask,
                                                              const float* __restrict__ lnw,
                                                              const float* __restrict__ lnb, float eps,
                                                              const TC* __restrict__ w4, TC* __restrict__ planes,
                                                              int B, int N, int Np, int outgoing) {
-  constexpr int BM = trimul_bm<TC>();
+  constexpr int BM = BM_;
   constexpr int NT = trimul_nt<C>();
   constexpr int LDA = C + lds_pad<TC>();
   constexpr int SLD = BM + lds_pad<TC>();
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(trimul_nt<C>()) void trimul_project_kernel(const TZ
   int wrow0[4 * CBW];
 #pragma unroll
   for (int j = 0; j < 4 * CBW; ++j) wrow0[j] = (w * CBW + j / 4) * 64 + (j % 4) * 16;
-  gemm16_lds_x_w<TC, C, RB, 4 * CBW>(acc, A, LDA, 0, w4, C, wrow0);
+  if (line < N && t0 < N) gemm16_lds_x_w<TC, C, RB, 4 * CBW>(acc, A, LDA, 0, w4, C, wrow0);
   __syncthreads();  // A is dead; its LDS becomes the staging tile S [2][C][SLD]
 
 #pragma unroll
@@ -1822,9 +1823,18 @@ int trimul_launch(const void* z, const float* mask, const float* lniw, const flo
                                                                    (const bf16*)w4, (bf16*)planes, B, N, Np,
                                                                    outgoing);
       (void)grid;
-    } else
-      trimul_project_kernel<TZ, TC, C><<<grid, trimul_nt<C>(), 0, s>>>((const TZ*)z, mask, lniw, lnib, eps_in, (const TC*)w4,
-                                                            planes, B, N, Np, outgoing);
+    } else {
+      // fp32: while 32-position blocks leave CUs idle, blocks of 16 (each streams the same
+      // weights, half the products): K1A_FIG
+      constexpr bool kSmall = sizeof(TC) == 4 && C <= 128;
+      if (kSmall && (long)B * N * ((N + BM - 1) / BM) <= pf::cu_count())
+        trimul_project_kernel<TZ, TC, C, true, kSmall ? 16 : BM>
+            <<<dim3(Np / 16, Np, B), trimul_nt<C>(), 0, s>>>((const TZ*)z, mask, lniw, lnib, eps_in, (const TC*)w4,
+                                                             planes, B, N, Np, outgoing);
+      else
+        trimul_project_kernel<TZ, TC, C><<<grid, trimul_nt<C>(), 0, s>>>(
+            (const TZ*)z, mask, lniw, lnib, eps_in, (const TC*)w4, planes, B, N, Np, outgoing);
+    }
     timer_trimul_project.stop();
     if (int e = pf::check_launch("trimul_project")) return e;
   }
