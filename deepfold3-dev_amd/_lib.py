@@ -47,6 +47,7 @@ SIGNATURES: dict[str, tuple] = {
     "pf_trimul_pack_weights": (_i, [_vp, _vp, _i, _vp, _i, _i, _vp]),
     "pf_trimul_train_pack_weights": (_i, [_vp, _vp, _i, _vp, _i, _i, _vp]),
     "pf_trimul_train_fwd": (_i, [_vp] * 3 + [_vp, _vp, _f, _vp, _vp] + [_i] * 6 + [_vp, _sz, _vp, _vp]),
+    "pf_trimul_vjp_pack": (_i, [_vp] * 3 + [_i, _i, _vp, _vp]),
     "pf_trimul_output_vjp_workspace_bytes": (_sz, [_i, _i, _i, _i]),
     "pf_trimul_output_vjp": (_i, [_vp] * 5 + [_f] + [_vp] * 4 + [_i] * 5 + [_vp] * 8 + [_sz, _vp]),
     "pf_trimul_project_vjp": (_i, [_vp] * 6 + [_i] * 6 + [_vp] * 4),

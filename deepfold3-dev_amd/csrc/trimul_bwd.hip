@@ -1074,6 +1074,23 @@ __global__ __launch_bounds__(256) void plane_transpose_kernel(const T* __restric
   }
 }
 
+// out = Wo^T [C][C] | Wog^T [C][C] | W4^T [C][4C]: the VJPs' transposed weights in one launch
+// (6 C^2 elements, all in L2: latency, 3 us).
+template <class T>
+__global__ __launch_bounds__(256) void vjp_pack_kernel(const T* __restrict__ wo, const T* __restrict__ wog,
+                                                       const T* __restrict__ w4, T* __restrict__ out, int C) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int cc = C * C;
+  if (i >= 6 * cc) return;
+  if (i < 2 * cc) {
+    const int j = i < cc ? i : i - cc;
+    out[i] = (i < cc ? wo : wog)[(j % C) * C + j / C];
+  } else {
+    const int j = i - 2 * cc;
+    out[i] = w4[(j % (4 * C)) * C + j / (4 * C)];
+  }
+}
+
 template <class TC, int C>
 size_t out_vjp_partials(int B, int N) {
   const int Np = pf::pad128(N);
@@ -1167,6 +1184,22 @@ bool vjp_args_ok(int B, int N, int C, int xdtype, int cdtype) {
 }  // namespace
 
 extern "C" {
+
+int pf_trimul_vjp_pack(const void* w_out, const void* w_out_gate, const void* w_packed, int C, int dtype, void* out,
+                       void* stream) {
+  PF_REQUIRE(w_out && w_out_gate && w_packed && out, PF_ERR_INVALID_ARG, "pf_trimul_vjp_pack: null pointer");
+  PF_REQUIRE((C == 64 || C == 128 || C == 256) && (dtype == PF_F32 || dtype == PF_BF16), PF_ERR_UNSUPPORTED,
+             "pf_trimul_vjp_pack: C=%d dtype %d", C, dtype);
+  hipStream_t s = pf::as_stream(stream);
+  const unsigned grid = (unsigned)(6 * C * C / 256);
+  if (dtype == PF_F32)
+    vjp_pack_kernel<float><<<grid, 256, 0, s>>>((const float*)w_out, (const float*)w_out_gate, (const float*)w_packed,
+                                                (float*)out, C);
+  else
+    vjp_pack_kernel<bf16><<<grid, 256, 0, s>>>((const bf16*)w_out, (const bf16*)w_out_gate, (const bf16*)w_packed,
+                                               (bf16*)out, C);
+  return pf::check_launch("pf_trimul_vjp_pack");
+}
 
 size_t pf_trimul_output_vjp_workspace_bytes(int B, int N, int C, int cdtype) {
   if (B <= 0 || N <= 0 || (cdtype != PF_F32 && cdtype != PF_BF16)) return 0;

@@ -671,7 +671,9 @@ class FusedTriMulFunction(torch.autograd.Function):
         dlnw, dlnb = (torch.empty(C, dtype=torch.float32, device=dev) for _ in range(2))
         ws_bytes = _lib.lib().pf_trimul_output_vjp_workspace_bytes(B, N, C, code_c)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-        wot, wogt = wo.t().contiguous(), wog.t().contiguous()
+        wt = torch.empty(6 * C * C, dtype=cdt, device=dev)  # Wo^T, Wog^T, W4^T
+        _lib.call("pf_trimul_vjp_pack", wo.data_ptr(), wog.data_ptr(), w4.data_ptr(), C, code_c, wt.data_ptr(), stream)
+        wot, wogt, w4t = wt[: C * C], wt[C * C : 2 * C * C], wt[2 * C * C :]
         args = (
             g.data_ptr(), pl[2].data_ptr(), xc.data_ptr(), lnow.data_ptr(), _lib.ptr(lnob), ctx.eps, wo.data_ptr(),
             wog.data_ptr(), wot.data_ptr(), wogt.data_ptr(), B, N, C, code_x, code_c, gp.data_ptr(), gg.data_ptr(),
@@ -711,7 +713,6 @@ class FusedTriMulFunction(torch.autograd.Function):
         gpg = torch.empty((M, 4 * C), dtype=cdt, device=dev)  # token-major, the kernel's walk order
         xw = None if ctx.outgoing else torch.empty((M, C), dtype=cdt, device=dev)  # x in that order
         dx = torch.empty_like(xc)
-        w4t = w4.t().contiguous()
         _lib.call(
             "pf_trimul_project_vjp", dpl.data_ptr(), xc.data_ptr(), m.data_ptr(), w4.data_ptr(), w4t.data_ptr(),
             gx.data_ptr(), B, N, C, int(ctx.outgoing), code_x, code_c, gpg.data_ptr(), _lib.ptr(xw), dx.data_ptr(),
@@ -720,8 +721,9 @@ class FusedTriMulFunction(torch.autograd.Function):
         del dpl, gx
         cb = 32 if (cdt == torch.bfloat16 and C == 128) else 16  # channel blocks of the packed rows
         dw4 = _weight_grad_tm(gpg, xb if xw is None else xw).view(C // cb, 4, cb, C)  # rows 4 cb j + cb kind + r
-        d_proj = torch.cat([dw4[:, 0].reshape(C, C), dw4[:, 2].reshape(C, C)])
-        d_gate = torch.cat([dw4[:, 1].reshape(C, C), dw4[:, 3].reshape(C, C)])
+        # kinds a proj, a gate, b proj, b gate; block order is all of a, then all of b
+        d_proj = dw4[:, 0::2].transpose(0, 1).reshape(2 * C, C)
+        d_gate = dw4[:, 1::2].transpose(0, 1).reshape(2 * C, C)
         dt = ctx.dtypes
         return (dx.to(dt[0]), None, d_gate.to(dt[1]), d_proj.to(dt[2]), dlnw.to(dt[3]),
                 None if dt[4] is None else dlnb.to(dt[4]), d_out.to(dt[5]), d_out_gate.to(dt[6]), None, None,

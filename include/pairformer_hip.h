@@ -188,6 +188,10 @@ int pf_trimul_train_fwd(const void* x, const float* mask, const void* w_packed, 
                         const float* ln_out_b, float eps_out, const void* w_out, const void* w_out_gate, int B, int N,
                         int C, int outgoing, int xdtype, int cdtype, void* planes, size_t planes_bytes, void* out,
                         void* stream);
+/* out [6 C C] = w_out^T [C, C] | w_out_gate^T [C, C] | w_packed^T [C, 4C], all in dtype: the
+ * transposed weights that the two VJPs take. */
+int pf_trimul_vjp_pack(const void* w_out, const void* w_out_gate, const void* w_packed, int C, int dtype, void* out,
+                       void* stream);
 size_t pf_trimul_output_vjp_workspace_bytes(int B, int N, int C, int cdtype);
 int pf_trimul_output_vjp(const void* g, const void* X, const void* x, const float* ln_out_w, const float* ln_out_b,
                          float eps_out, const void* w_out, const void* w_out_gate, const void* w_out_t,
